@@ -337,8 +337,17 @@ hipError_t launch_d3q39_from_fp64(const Box& b, const double* src, void* dst, in
 // stride in elements) <-> [ncomp][n] in the box's node order
 hipError_t launch_fab_gather(const double* fab, int ghost, int64_t cstride, const Box& b,
                              int ncomp, double* dense, hipStream_t s);
-hipError_t launch_fab_scatter(const double* dense, const Box& b, int ncomp, int ghost,
-                              int64_t cstride, double* fab, hipStream_t s);
+// the same array <-> [ncomp][n] in a storage form holding value - ref[comp]
+// (float if fp32, else double); the import fills one or two buffers.  ncomp
+// 27, 39 or 13.
+struct FabRef {
+  double v[39];
+};
+hipError_t launch_fab_import(const double* fab, int ghost, int64_t cstride, const Box& b,
+                             int ncomp, const FabRef& ref, int fp32, void* dst0, void* dst1,
+                             hipStream_t s);
+hipError_t launch_fab_export(const void* src, const Box& b, int ncomp, const FabRef& ref,
+                             int fp32, int ghost, int64_t cstride, double* fab, hipStream_t s);
 hipError_t launch_blank_gather(const int32_t* code, int ghost, const Box& b, int32_t* blank,
                                hipStream_t s);
 hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);

@@ -3049,34 +3049,33 @@ int uclbs_import_fab(void* ctx, int lvl, int field, const double* fab, int ghost
                      int64_t comp_stride) {
   Ctx* c = static_cast<Ctx*>(ctx);
   Level* L;
+// what the storage form of a population field holds less of, per component:
+// the lattice weights (D3Q27) or the reference equilibrium (D3Q39) in FP32,
+// nothing in FP64
+uclbs::FabRef fab_ref(const Ctx* c, int field) {
+  uclbs::FabRef r{};
+  if (c->cfg.lattice == UCLBS_LATTICE_D3Q39) {
+    const double* v = field == UCLBS_FIELD_G ? c->ref39.g : c->ref39.f;
+    for (int i = 0; i < uclbs::Q39; ++i) r.v[i] = v[i];
+  } else if (c->cfg.precision == UCLBS_PREC_FP32_SHIFTED) {
+    for (int i = 0; i < 27; ++i) r.v[i] = uclbs::W27[i];
+  }
+  return r;
+}
+
   int ncomp = 0;
   int rc = fab_args(c, lvl, field, fab, ghost, comp_stride, &L, &ncomp);
   if (rc) return rc;
-  const bool fp32 = c->cfg.precision == UCLBS_PREC_FP32_SHIFTED;
-  hipError_t e = hipSuccess;
+  hipError_t e;
   if (field == UCLBS_FIELD_LM) {
-    e = uclbs::launch_fab_gather(fab, ghost, comp_stride, L->box, ncomp, L->lm, c->stream);
+    e = uclbs::launch_fab_import(fab, ghost, comp_stride, L->box, ncomp, uclbs::FabRef{}, 0, L->lm,
+                                 nullptr, c->stream);
   } else {
-    double* tmp = nullptr;
-    e = hipMalloc(&tmp, (size_t)L->box.n * ncomp * sizeof(double));
-    if (e == hipSuccess)
-      e = uclbs::launch_fab_gather(fab, ghost, comp_stride, L->box, ncomp, tmp, c->stream);
-    void* cur = field == UCLBS_FIELD_F ? L->f[L->cur] : L->g[L->cur];
-    void* other = field == UCLBS_FIELD_F ? L->f[1 - L->cur] : L->g[1 - L->cur];
-    if (e == hipSuccess) {
-      if (c->cfg.lattice == UCLBS_LATTICE_D3Q27)
-        e = uclbs::launch_d3q27_from_fp64(L->box, tmp, cur, fp32, c->stream);
-      else
-        e = uclbs::launch_d3q39_from_fp64(L->box, tmp, cur, fp32,
-                                          c->d_ref39 + (field == UCLBS_FIELD_G ? uclbs::Q39 : 0),
-                                          c->stream);
-    }
     // the other buffer mirrors the imported one (nodes no kernel writes)
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(other, cur, level_bytes(c, L) / q_of(c) * ncomp,
-                         hipMemcpyDeviceToDevice, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (tmp) (void)hipFree(tmp);
+    void** buf = field == UCLBS_FIELD_F ? L->f : L->g;
+    e = uclbs::launch_fab_import(fab, ghost, comp_stride, L->box, ncomp, fab_ref(c, field),
+                                 c->cfg.precision == UCLBS_PREC_FP32_SHIFTED, buf[L->cur],
+                                 buf[1 - L->cur], c->stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return set_err(UCLBS_E_HIP, "import_fab: %s", hipGetErrorString(e));
@@ -3090,27 +3089,15 @@ int uclbs_export_fab(void* ctx, int lvl, int field, double* fab, int ghost, int6
   int ncomp = 0;
   int rc = fab_args(c, lvl, field, fab, ghost, comp_stride, &L, &ncomp);
   if (rc) return rc;
-  const bool fp32 = c->cfg.precision == UCLBS_PREC_FP32_SHIFTED;
-  hipError_t e = hipSuccess;
-  if (field == UCLBS_FIELD_LM) {
-    e = uclbs::launch_fab_scatter(L->lm, L->box, ncomp, ghost, comp_stride, fab, c->stream);
-  } else {
-    double* tmp = nullptr;
-    e = hipMalloc(&tmp, (size_t)L->box.n * ncomp * sizeof(double));
-    const void* cur = field == UCLBS_FIELD_F ? L->f[L->cur] : L->g[L->cur];
-    if (e == hipSuccess) {
-      if (c->cfg.lattice == UCLBS_LATTICE_D3Q27)
-        e = uclbs::launch_d3q27_to_fp64(L->box, cur, tmp, fp32, c->stream);
-      else
-        e = uclbs::launch_d3q39_to_fp64(L->box, cur, tmp, fp32,
-                                        c->d_ref39 + (field == UCLBS_FIELD_G ? uclbs::Q39 : 0),
-                                        c->stream);
-    }
-    if (e == hipSuccess)
-      e = uclbs::launch_fab_scatter(tmp, L->box, ncomp, ghost, comp_stride, fab, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (tmp) (void)hipFree(tmp);
-  }
+  hipError_t e;
+  if (field == UCLBS_FIELD_LM)
+    e = uclbs::launch_fab_export(L->lm, L->box, ncomp, uclbs::FabRef{}, 0, ghost, comp_stride, fab,
+                                 c->stream);
+  else
+    e = uclbs::launch_fab_export(field == UCLBS_FIELD_F ? L->f[L->cur] : L->g[L->cur], L->box,
+                                 ncomp, fab_ref(c, field),
+                                 c->cfg.precision == UCLBS_PREC_FP32_SHIFTED, ghost, comp_stride,
+                                 fab, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return set_err(UCLBS_E_HIP, "export_fab: %s", hipGetErrorString(e));
   return UCLBS_OK;
