@@ -3043,12 +3043,6 @@ int fab_args(Ctx* c, int lvl, int field, const void* fab, int ghost, int64_t cst
   return UCLBS_OK;
 }
 
-}  // namespace
-
-int uclbs_import_fab(void* ctx, int lvl, int field, const double* fab, int ghost,
-                     int64_t comp_stride) {
-  Ctx* c = static_cast<Ctx*>(ctx);
-  Level* L;
 // what the storage form of a population field holds less of, per component:
 // the lattice weights (D3Q27) or the reference equilibrium (D3Q39) in FP32,
 // nothing in FP64
@@ -3063,6 +3057,12 @@ uclbs::FabRef fab_ref(const Ctx* c, int field) {
   return r;
 }
 
+}  // namespace
+
+int uclbs_import_fab(void* ctx, int lvl, int field, const double* fab, int ghost,
+                     int64_t comp_stride) {
+  Ctx* c = static_cast<Ctx*>(ctx);
+  Level* L;
   int ncomp = 0;
   int rc = fab_args(c, lvl, field, fab, ghost, comp_stride, &L, &ncomp);
   if (rc) return rc;
