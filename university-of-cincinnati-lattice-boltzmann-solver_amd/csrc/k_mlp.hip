@@ -30,16 +30,6 @@ constexpr int oW1 = 0, oB1 = oW1 + kIn * kH, oW2 = oB1 + kH, oB2 = oW2 + kH * kH
               oW3 = oB2 + kH, oB3 = oW3 + kH * kH, oW4 = oB3 + kH, oB4 = oW4 + kH;
 static_assert(oB4 + 1 == kMlpParams, "parameter count");
 
-__device__ __forceinline__ float gelu(float x) {
-  const float c = 0.7978845608028654f;  // sqrt(2 / pi)
-  return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
-}
-__device__ __forceinline__ float gelu_grad(float x) {
-  const float c = 0.7978845608028654f;
-  const float t = tanhf(c * (x + 0.044715f * x * x * x));
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * x * x);
-}
-
 // The 12 features of a node from its pre-collision shifted populations, in
 // FP32 (they feed a BF16 network; the moments and equilibrium behind D are the
 // streaming kernel's FP64-summed ones).  Returns m = max|x| (0 for a node at
@@ -234,132 +224,382 @@ __global__ void k_collect_targets(const double* __restrict__ alpha, const unsign
 }
 
 // ---- training (FP32) -------------------------------------------------------
-// Z[b][o] = sum_k A[b][k] W[k][o] + bias[o]; Aout = gelu(Z) (or Z)
-__global__ void k_fwd_layer(const float* __restrict__ A, int K, const float* __restrict__ W,
-                            const float* __restrict__ bias, int O, int B, int act,
-                            float* __restrict__ Z, float* __restrict__ Aout) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B * O) return;
-  const int r = t / O, o = t % O;
-  float s = bias[o];
-  for (int k = 0; k < K; ++k) s = fmaf(A[r * K + k], W[k * O + o], s);
-  Z[t] = s;
-  Aout[t] = act ? gelu(s) : s;
+// One launch takes a batch through the network and back, a second adds the
+// weight gradients up (and, in training, applies Adam); activations stay in
+// registers and LDS.  Launch per layer and direction, the same step took 18
+// launches whose threads each ran a serial loop over a row or a chunk of rows.
+//
+// A block of four wavefronts holds 32 rows; wavefront w computes 16 of them
+// (w & 1) and 32 of a layer's 64 outputs (w >> 1), so that a batch of 8,192
+// gives each of the 256 CUs one block.  All products run on
+// v_mfma_f32_16x16x4_f32 (FP32 in, FP32 accumulation): A lane l = row l % 16,
+// k = l / 16; B lane l = column l % 16, the same k; D lane l = column l % 16,
+// rows 4 (l / 16) + 0..3.  Layers are computed transposed, O^T = W^T X^T, and
+// MFMA step s of a 16-wide chunk takes k = 4 (l / 16) + s for both operands, so
+// that a D tile's rows are the next product's k.  Every tile lives in LDS as
+// [feature][row] (pitch kTp): the forward and backward products read it by
+// column, the weight gradients, which contract over the rows, by float4.  Each
+// wavefront reads its half of a weight matrix once, into registers.
+// Bound by the FP32 matrix rate and the chain of seven layer products with a
+// barrier after each: 206 MFMA a wavefront (2.8 us at 32 cycles each).
+constexpr int kTrainRows = 32;
+constexpr int kTp = kTrainRows + 4;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// dZ of the output layer and the batch loss: dZ = (yhat - y) / B, loss = 0.5 mean r^2
-__global__ void k_out_grad(const float* __restrict__ yhat, const float* __restrict__ y,
-                           const unsigned* __restrict__ idx, int B, float* __restrict__ dZ,
-                           double* __restrict__ loss) {
-  __shared__ double red[256];
-  double acc = 0.0;
-  for (int r = threadIdx.x; r < B; r += blockDim.x) {
-    const float yt = idx ? y[idx[r]] : y[r];
-    const float d = yhat[r] - yt;
-    dZ[r] = d / (float)B;
-    acc += 0.5 * (double)d * d;
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *loss = red[0] / B;
+// h = gelu(z), gp = gelu'(z) over one tanh
+__device__ __forceinline__ float gelu_both(float x, float& gp) {
+  const float c = 0.7978845608028654f;
+  const float t = tanhf(c * (x + 0.044715f * x * x * x));
+  gp = 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * x * x);
+  return 0.5f * x * (1.0f + t);
 }
 
-// Weight gradients gW[k][o] = sum_r A[r][k] dZ[r][o] and gb[o] = sum_r dZ[r][o]
-// in two deterministic passes: each block of the first sums one chunk of
-// kRowChunk rows for 256 weights (one weight per thread), the second adds the
-// chunk sums in chunk order.
-constexpr int kRowChunk = 256;
-__global__ void k_bwd_weights_part(const float* __restrict__ A, int K, const float* __restrict__ dZ,
-                                   int O, int B, float* __restrict__ part) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = K * O + O;
-  if (t >= n) return;
-  const int r0 = (int)blockIdx.y * kRowChunk, r1 = min(B, r0 + kRowChunk);
-  float s = 0.0f;
-  if (t < K * O) {
-    const int k = t / O, o = t % O;
-    for (int r = r0; r < r1; ++r) s = fmaf(A[r * K + k], dZ[r * O + o], s);
-  } else {
-    const int o = t - K * O;
-    for (int r = r0; r < r1; ++r) s += dZ[r * O + o];
-  }
-  part[(size_t)blockIdx.y * n + t] = s;
-}
-
-__global__ void k_bwd_weights_sum(const float* __restrict__ part, int K, int O, int nc,
-                                  float* __restrict__ gW, float* __restrict__ gb) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = K * O + O;
-  if (t >= n) return;
-  float s = 0.0f;
-  for (int c = 0; c < nc; ++c) s += part[(size_t)c * n + t];
-  if (t < K * O) gW[t] = s;
-  else gb[t - K * O] = s;
-}
-
-// dZprev[b][k] = (sum_o dZ[b][o] W[k][o]) * gelu'(Zprev[b][k])
-__global__ void k_bwd_input(const float* __restrict__ dZ, int O, const float* __restrict__ W,
-                            const float* __restrict__ Zprev, int K, int B,
-                            float* __restrict__ dZprev) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B * K) return;
-  const int r = t / K, k = t % K;
-  float s = 0.0f;
-  for (int o = 0; o < O; ++o) s = fmaf(dZ[r * O + o], W[k * O + o], s);
-  dZprev[t] = s * gelu_grad(Zprev[t]);
-}
-
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, int n, float lr, float c1, float c2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const float gk = g[k];
-  const float mk = 0.9f * m[k] + 0.1f * gk;
-  const float vk = 0.999f * v[k] + 0.001f * gk * gk;
-  m[k] = mk;
-  v[k] = vk;
-  p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
-}
-
-// gather a random batch of samples (Philox4x32-10 indices, with replacement)
-__global__ void k_gather(const float* __restrict__ X, unsigned long long n, uint64_t seed,
-                         uint64_t step, int B, float* __restrict__ Xb, unsigned* __restrict__ idx) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= B) return;
-  uint32_t c[4] = {(uint32_t)r, (uint32_t)step, (uint32_t)(step >> 32), 0x6d6c70u};
-  philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-  const unsigned long long k = (((unsigned long long)c[0] << 32) | c[1]) % n;
-  idx[r] = (unsigned)k;
+// A operand of a forward product: W^T[o = 16 ot + l % 16][k], 16 k-steps
+__device__ __forceinline__ void load_fwd(const float* __restrict__ W, int ot, int c16, int g,
+                                         float (&a)[16]) {
 #pragma unroll
-  for (int j = 0; j < kIn; ++j) Xb[r * kIn + j] = X[k * kIn + j];
+  for (int t = 0; t < 16; ++t) a[t] = W[(16 * (t / 4) + 4 * g + t % 4) * kH + 16 * ot + c16];
+}
+// A operand of a backward product: W[k = 16 kt + l % 16][o], 16 o-steps
+__device__ __forceinline__ void load_bwd(const float* __restrict__ W, int kt, int c16, int g,
+                                         f32x4 (&a)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    a[q] = *reinterpret_cast<const f32x4*>(W + (16 * kt + c16) * kH + 16 * q + 4 * g);
 }
 
-// mean and standard deviation of the targets (one block, FP64)
-__global__ void k_moments(const float* __restrict__ y, unsigned long long n, double* __restrict__ out) {
-  __shared__ double s1[256], s2[256];
-  double a = 0.0, b = 0.0;
-  for (unsigned long long k = threadIdx.x; k < n; k += blockDim.x) {
-    a += y[k];
-    b += (double)y[k] * y[k];
+enum { kRowsForward = 0, kRowsGrad = 1, kRowsGather = 2 };
+
+// kRowsForward: yhat of rows 0..B-1 of X.  kRowsGrad: the block's sums of the
+// weight gradients over its rows into part[block][kMlpParams] and of the loss
+// into lpart[block].  kRowsGather: the same over rows drawn from n samples
+// (Philox4x32-10 indices, with replacement).
+template <int kMode>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_mlp_rows(const float* __restrict__ P,
+                                                  const float* __restrict__ X,
+                                                  const float* __restrict__ y, int B,
+                                                  unsigned long long n, uint64_t seed,
+                                                  uint64_t step, float* __restrict__ part,
+                                                  double* __restrict__ lpart,
+                                                  float* __restrict__ yhat) {
+  constexpr bool kBack = kMode != kRowsForward;
+  __shared__ __attribute__((aligned(16))) float Xs[16][kTp];
+  __shared__ __attribute__((aligned(16))) float H[3][kH][kTp];
+  __shared__ __attribute__((aligned(16))) float D[kBack ? 3 : 1][kBack ? kH : 1][kTp];
+  __shared__ float ysum[2][kTrainRows];
+  __shared__ __attribute__((aligned(16))) float dz[kTrainRows];
+  __shared__ unsigned sidx[kTrainRows];
+  const int tid = (int)threadIdx.x, l = tid % 64, w = tid / 64;
+  const int c16 = l % 16, g = l / 16;
+  const int nt = w & 1, hf = w >> 1;  // rows 16 nt .., output tiles 2 hf, 2 hf + 1
+  const int col = 16 * nt + c16;      // this lane's row of the tile
+  const float *W1 = P + oW1, *W2 = P + oW2, *W3 = P + oW3;
+
+  float a1[2][3], a2[2][16], a3[2][16];
+  f32x4 b1[2], b2[2], b3[2], w4[2];
+#pragma unroll
+  for (int o = 0; o < 2; ++o) {
+    const int ot = 2 * hf + o;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) a1[o][s] = W1[(4 * s + g) * kH + 16 * ot + c16];
+    load_fwd(W2, ot, c16, g, a2[o]);
+    load_fwd(W3, ot, c16, g, a3[o]);
+    const int r = 16 * ot + 4 * g;
+    b1[o] = *reinterpret_cast<const f32x4*>(P + oB1 + r);
+    b2[o] = *reinterpret_cast<const f32x4*>(P + oB2 + r);
+    b3[o] = *reinterpret_cast<const f32x4*>(P + oB3 + r);
+    w4[o] = *reinterpret_cast<const f32x4*>(P + oW4 + r);
   }
-  s1[threadIdx.x] = a;
-  s2[threadIdx.x] = b;
+  const float b4 = P[oB4];
+
+  // sums over this block's tiles: gW3, gW2 (k-tile w, the four o-tiles), gW1
+  // (o-tile w), one entry of gW4 / gb3 / gb2 / gb1 a thread, gb4 and the loss
+  f32x4 s3[4], s2[4], s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int o = 0; o < 4; ++o) s3[o] = s2[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float sv = 0.0f, sb4 = 0.0f;
+  double sl = 0.0;
+
+  const int ntiles = (B + kTrainRows - 1) / kTrainRows;
+  for (int tile = (int)blockIdx.x; tile < ntiles; tile += (int)gridDim.x) {
+    const int r0 = tile * kTrainRows;
+    float yt = 0.0f;
+    if (tid < kTrainRows) {
+      const int r = r0 + tid;
+      unsigned k = (unsigned)(r < B ? r : 0);
+      if constexpr (kMode == kRowsGather) {
+        uint32_t c[4] = {(uint32_t)r, (uint32_t)step, (uint32_t)(step >> 32), 0x6d6c70u};
+        philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+        k = (unsigned)((((unsigned long long)c[0] << 32) | c[1]) % n);
+      }
+      sidx[tid] = k;
+      if constexpr (kBack) yt = y[k];
+    }
+    __syncthreads();
+    if (tid < 4 * kTrainRows) {
+      const int r = tid / 4, q = tid % 4;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (q < 3 && r0 + r < B)
+        v = *reinterpret_cast<const f32x4*>(X + (size_t)sidx[r] * kIn + 4 * q);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) Xs[4 * q + j][r] = v[j];
+    }
+    __syncthreads();
+
+    f32x4 p1[2], p2[2], p3[2];  // gelu' of the three layers at (16 ot + 4 g + j, col)
+    auto act = [&](float (*Hl)[kTp], const f32x4 (&z)[2], f32x4 (&p)[2]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float gp;
+          Hl[16 * (2 * hf + o) + 4 * g + j][col] = gelu_both(z[o][j], gp);
+          p[o][j] = gp;
+        }
+    };
+    f32x4 z[2] = {b1[0], b1[1]};
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const float b = Xs[4 * s + g][col];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) z[o] = mfma4(a1[o][s], b, z[o]);
+    }
+    act(H[0], z, p1);
+    __syncthreads();
+    auto layer = [&](const float (*Hl)[kTp], const float (&a)[2][16], const f32x4 (&b)[2]) __attribute__((always_inline)) {
+      z[0] = b[0];
+      z[1] = b[1];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const float h = Hl[16 * (t / 4) + 4 * g + t % 4][col];
+#pragma unroll
+        for (int o = 0; o < 2; ++o) z[o] = mfma4(a[o][t], h, z[o]);
+      }
+    };
+    layer(H[0], a2, b2);
+    act(H[1], z, p2);
+    __syncthreads();
+    layer(H[1], a3, b3);
+    float yp = 0.0f;
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float gp;
+        const float h = gelu_both(z[o][j], gp);
+        p3[o][j] = gp;
+        if constexpr (kBack) H[2][16 * (2 * hf + o) + 4 * g + j][col] = h;
+        yp = fmaf(h, w4[o][j], yp);
+      }
+    yp += __shfl_xor(yp, 16);
+    yp += __shfl_xor(yp, 32);
+    if (g == 0) ysum[hf][col] = yp;
+    __syncthreads();
+    if (tid < kTrainRows) {
+      const float yh = (ysum[0][tid] + ysum[1][tid]) + b4;
+      const bool in = r0 + tid < B;
+      if constexpr (kBack) {
+        const float d = in ? yh - yt : 0.0f;
+        const float v = d / (float)B;
+        dz[tid] = v;
+        sb4 += v;
+        sl += 0.5 * (double)d * d;
+      } else if (in) {
+        yhat[r0 + tid] = yh;
+      }
+    }
+    __syncthreads();
+    if constexpr (kBack) {
+      f32x4 w3[2][4], w2[2][4];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        load_bwd(W3, 2 * hf + o, c16, g, w3[o]);
+        load_bwd(W2, 2 * hf + o, c16, g, w2[o]);
+      }
+      {
+        const float d4 = dz[col];
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            D[2][16 * (2 * hf + o) + 4 * g + j][col] = (d4 * w4[o][j]) * p3[o][j];
+      }
+      __syncthreads();
+      auto back = [&](const float (*Dl)[kTp], const f32x4 (&a)[2][4], const f32x4 (&p)[2],
+                      float (*Dp)[kTp]) __attribute__((always_inline)) {
+        z[0] = z[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const float d = Dl[16 * q + 4 * g + s][col];
+#pragma unroll
+            for (int o = 0; o < 2; ++o) z[o] = mfma4(a[o][q][s], d, z[o]);
+          }
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) Dp[16 * (2 * hf + o) + 4 * g + j][col] = z[o][j] * p[o][j];
+      };
+      back(D[2], w3, p2, D[1]);
+      __syncthreads();
+      back(D[1], w2, p1, D[0]);
+      __syncthreads();
+      // weight gradients, contracted over the 32 rows
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int rr = 16 * q + 4 * g;
+        const f32x4 h2 = *reinterpret_cast<const f32x4*>(&H[1][16 * w + c16][rr]);
+        const f32x4 h1 = *reinterpret_cast<const f32x4*>(&H[0][16 * w + c16][rr]);
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&Xs[c16][rr]);
+        const f32x4 d1 = *reinterpret_cast<const f32x4*>(&D[0][16 * w + c16][rr]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) s1 = mfma4(x[s], d1[s], s1);
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+          const f32x4 d3 = *reinterpret_cast<const f32x4*>(&D[2][16 * o + c16][rr]);
+          const f32x4 d2 = *reinterpret_cast<const f32x4*>(&D[1][16 * o + c16][rr]);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            s3[o] = mfma4(h2[s], d3[s], s3[o]);
+            s2[o] = mfma4(h1[s], d2[s], s2[o]);
+          }
+        }
+      }
+      // wavefront 0: gW4, 1: gb3, 2: gb2, 3: gb1, one feature a lane
+      const float* src = w == 0 ? &H[2][l][0] : &D[3 - w][l][0];
+#pragma unroll
+      for (int r = 0; r < kTrainRows; r += 4) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(src + r);
+        const f32x4 m = *reinterpret_cast<const f32x4*>(&dz[r]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sv = w == 0 ? fmaf(v[j], m[j], sv) : sv + v[j];
+      }
+      __syncthreads();
+    }
+  }
+  if constexpr (kBack) {
+    float* o = part + (size_t)blockIdx.x * kMlpParams;
+#pragma unroll
+    for (int ot = 0; ot < 4; ++ot)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        o[oW3 + (16 * w + 4 * g + j) * kH + 16 * ot + c16] = s3[ot][j];
+        o[oW2 + (16 * w + 4 * g + j) * kH + 16 * ot + c16] = s2[ot][j];
+      }
+    if (g < 3) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[oW1 + (4 * g + j) * kH + 16 * w + c16] = s1[j];
+    }
+    o[(w == 0 ? oW4 : w == 1 ? oB3 : w == 2 ? oB2 : oB1) + l] = sv;
+    if (w == 0) {
+      // lanes 0..31 hold the rows' sums, the others zero
+#pragma unroll
+      for (int d = 16; d > 0; d >>= 1) {
+        sb4 += __shfl_xor(sb4, d);
+        sl += __shfl_xor(sl, d);
+      }
+      if (l == 0) {
+        o[oB4] = sb4;
+        lpart[blockIdx.x] = sl;
+      }
+    }
+  }
+}
+
+// The gradient as the sum of nb blocks' parts, eight slices of the blocks a
+// weight (a fixed order, so the result is the same from run to run), and the
+// mean loss.  kAdam: applied to the parameters at once; else stored in g.
+// 32 weights a block: a slice's loads are 128 B rows of part.
+template <bool kAdam>
+__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ part,
+                                                    const double* __restrict__ lpart, int nb,
+                                                    int B, float* __restrict__ gout,
+                                                    double* __restrict__ loss,
+                                                    float* __restrict__ p, float* __restrict__ m,
+                                                    float* __restrict__ v, float lr, float c1,
+                                                    float c2) {
+  __shared__ float red[8][32];
+  __shared__ double lred[256];
+  const int t = (int)threadIdx.x, c = t % 32, sl = t / 32;
+  const int k = (int)blockIdx.x * 32 + c;
+  float s = 0.0f;
+  if (k < kMlpParams) {
+    const int per = (nb + 7) / 8, lo = sl * per, hi = min(nb, lo + per);
+    for (int b = lo; b < hi; ++b) s += part[(size_t)b * kMlpParams + k];
+  }
+  red[sl][c] = s;
+  if (blockIdx.x == 0) {
+    double a = 0.0;
+    for (int b = t; b < nb; b += 256) a += lpart[b];
+    lred[t] = a;
+    __syncthreads();
+    for (int d = 128; d > 0; d >>= 1) {
+      if (t < d) lred[t] += lred[t + d];
+      __syncthreads();
+    }
+    if (t == 0) *loss = lred[0] / B;
+  }
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      s1[threadIdx.x] += s1[threadIdx.x + s];
-      s2[threadIdx.x] += s2[threadIdx.x + s];
+  if (t >= 32 || k >= kMlpParams) return;
+  const float gk = ((red[0][c] + red[1][c]) + (red[2][c] + red[3][c])) +
+                   ((red[4][c] + red[5][c]) + (red[6][c] + red[7][c]));
+  if constexpr (kAdam) {
+    const float mk = 0.9f * m[k] + 0.1f * gk;
+    const float vk = 0.999f * v[k] + 0.001f * gk * gk;
+    m[k] = mk;
+    v[k] = vk;
+    p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
+  } else {
+    gout[k] = gk;
+  }
+}
+
+// mean and standard deviation of the targets in FP64: a block's sums, then
+// one block over the blocks (one block over all of 786k targets ran for 1.6 ms)
+constexpr int kMomentBlocks = 256;
+__device__ __forceinline__ void sum2_256(double& a, double& b) {
+  __shared__ double s1[256], s2[256];
+  const int t = (int)threadIdx.x;
+  s1[t] = a;
+  s2[t] = b;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) {
+      s1[t] += s1[t + s];
+      s2[t] += s2[t + s];
     }
     __syncthreads();
   }
+  a = s1[0];
+  b = s2[0];
+}
+__global__ __launch_bounds__(256) void k_moments_part(const float* __restrict__ y,
+                                                      unsigned long long n,
+                                                      double* __restrict__ sums) {
+  double a = 0.0, b = 0.0;
+  for (unsigned long long k = blockIdx.x * 256ull + threadIdx.x; k < n; k += gridDim.x * 256ull) {
+    a += y[k];
+    b += (double)y[k] * y[k];
+  }
+  sum2_256(a, b);
   if (threadIdx.x == 0) {
-    const double mean = s1[0] / (double)n;
+    sums[2 * blockIdx.x] = a;
+    sums[2 * blockIdx.x + 1] = b;
+  }
+}
+__global__ __launch_bounds__(256) void k_moments(const double* __restrict__ sums,
+                                                 unsigned long long n, double* __restrict__ out) {
+  double a = sums[2 * threadIdx.x], b = sums[2 * threadIdx.x + 1];
+  sum2_256(a, b);
+  if (threadIdx.x == 0) {
+    const double mean = a / (double)n;
     out[0] = mean;
-    out[1] = sqrt(fmax(s2[0] / (double)n - mean * mean, 1e-30));
+    out[1] = sqrt(fmax(b / (double)n - mean * mean, 1e-30));
   }
 }
 
@@ -377,7 +617,6 @@ __global__ void k_normalise(float* __restrict__ y, unsigned long long n, const d
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4;
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
 typedef __bf16 bf16v8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ bf16x8 cat8(bf16x4 a, bf16x4 b) {
   return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
@@ -606,62 +845,52 @@ hipError_t launch_mlp_targets(const double* alpha, MlpSamples& s, unsigned long 
   return hipGetLastError();
 }
 
-// forward + backward of one batch (X: B x 12, y: targets; idx maps rows into
-// y or is null); gradients into g (kMlpParams), loss into *loss
-hipError_t launch_mlp_loss_grad(const float* P, const float* X, const float* y,
-                                const unsigned* idx, int B, MlpWork& w, float* g, double* loss,
-                                hipStream_t st) {
-  const int T = 256;
-  auto nb = [&](int n) { return dim3((unsigned)((n + T - 1) / T)); };
-  const int nc = (B + kRowChunk - 1) / kRowChunk;
-  auto bwd_weights = [&](const float* A, int K, const float* dZ, int O, int Bn, float* gW, float* gb) {
-    const int n = K * O + O;
-    hipLaunchKernelGGL(k_bwd_weights_part, dim3((unsigned)((n + T - 1) / T), (unsigned)nc), dim3(T), 0,
-                       st, A, K, dZ, O, Bn, w.part);
-    hipLaunchKernelGGL(k_bwd_weights_sum, nb(n), dim3(T), 0, st, w.part, K, O, nc, gW, gb);
-  };
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, X, kIn, P + oW1, P + oB1, kH, B, 1, w.Z1, w.A1);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, w.A1, kH, P + oW2, P + oB2, kH, B, 1, w.Z2, w.A2);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, w.A2, kH, P + oW3, P + oB3, kH, B, 1, w.Z3, w.A3);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B), dim3(T), 0, st, w.A3, kH, P + oW4, P + oB4, 1, B, 0, w.Z4, w.A4);
-  hipLaunchKernelGGL(k_out_grad, dim3(1), dim3(256), 0, st, w.A4, y, idx, B, w.D4, loss);
-  bwd_weights(w.A3, kH, w.D4, 1, B, g + oW4, g + oB4);
-  hipLaunchKernelGGL(k_bwd_input, nb(B * kH), dim3(T), 0, st, w.D4, 1, P + oW4, w.Z3, kH, B, w.D3);
-  bwd_weights(w.A2, kH, w.D3, kH, B, g + oW3, g + oB3);
-  hipLaunchKernelGGL(k_bwd_input, nb(B * kH), dim3(T), 0, st, w.D3, kH, P + oW3, w.Z2, kH, B, w.D2);
-  bwd_weights(w.A1, kH, w.D2, kH, B, g + oW2, g + oB2);
-  hipLaunchKernelGGL(k_bwd_input, nb(B * kH), dim3(T), 0, st, w.D2, kH, P + oW2, w.Z1, kH, B, w.D1);
-  bwd_weights(X, kIn, w.D1, kH, B, g + oW1, g + oB1);
+int mlp_blocks(int B) {
+  // one block a CU (its weights and sums take 363 VGPRs, one wavefront a SIMD);
+  // a block strides over the tiles beyond and keeps its weights and sums
+  return std::min((B + kTrainRows - 1) / kTrainRows, 256);
+}
+
+// forward + backward of one batch (X: B x 12, y: B targets); gradients into g
+// (kMlpParams), loss into *loss
+hipError_t launch_mlp_loss_grad(const float* P, const float* X, const float* y, int B,
+                                const MlpWork& w, float* g, double* loss, hipStream_t st) {
+  const int nb = mlp_blocks(B);
+  hipLaunchKernelGGL(k_mlp_rows<kRowsGrad>, dim3(nb), dim3(256), 0, st, P, X, y, B, 0ull,
+                     (uint64_t)0, (uint64_t)0, w.part, w.loss, (float*)nullptr);
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 31) / 32), dim3(256), 0, st, w.part,
+                     w.loss, nb, B, g, loss, (float*)nullptr, (float*)nullptr, (float*)nullptr,
+                     0.0f, 0.0f, 0.0f);
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_forward_fp32(const float* P, const float* X, int B, MlpWork& w, float* yhat,
-                                   hipStream_t st) {
-  const int T = 256;
-  auto nb = [&](int n) { return dim3((unsigned)((n + T - 1) / T)); };
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, X, kIn, P + oW1, P + oB1, kH, B, 1, w.Z1, w.A1);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, w.A1, kH, P + oW2, P + oB2, kH, B, 1, w.Z2, w.A2);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B * kH), dim3(T), 0, st, w.A2, kH, P + oW3, P + oB3, kH, B, 1, w.Z3, w.A3);
-  hipLaunchKernelGGL(k_fwd_layer, nb(B), dim3(T), 0, st, w.A3, kH, P + oW4, P + oB4, 1, B, 0, w.Z4, yhat);
-  return hipGetLastError();
-}
-
-hipError_t launch_mlp_adam(float* P, const float* g, float* m, float* v, int t, float lr,
-                           hipStream_t st) {
+// training step t of Adam on a batch of B drawn from the n samples (X, y);
+// the batch's loss before the step into *loss
+hipError_t launch_mlp_train_step(float* P, float* m, float* v, const float* X, const float* y,
+                                 unsigned long long n, uint64_t seed, uint64_t step, int B, int t,
+                                 float lr, const MlpWork& w, double* loss, hipStream_t st) {
+  const int nb = mlp_blocks(B);
   const float c1 = 1.0f - powf(0.9f, (float)t), c2 = 1.0f - powf(0.999f, (float)t);
-  hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, P, g, m, v,
-                     kMlpParams, lr, c1, c2);
+  hipLaunchKernelGGL(k_mlp_rows<kRowsGather>, dim3(nb), dim3(256), 0, st, P, X, y, B, n, seed, step,
+                     w.part, w.loss, (float*)nullptr);
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 31) / 32), dim3(256), 0, st, w.part,
+                     w.loss, nb, B, (float*)nullptr, loss, P, m, v, lr, c1, c2);
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_gather(const float* X, unsigned long long n, uint64_t seed, uint64_t step,
-                             int B, float* Xb, unsigned* idx, hipStream_t st) {
-  hipLaunchKernelGGL(k_gather, dim3((B + 255) / 256), dim3(256), 0, st, X, n, seed, step, B, Xb, idx);
+hipError_t launch_mlp_forward_fp32(const float* P, const float* X, int B, float* yhat,
+                                   hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_rows<kRowsForward>, dim3(mlp_blocks(B)), dim3(256), 0, st, P, X,
+                     (const float*)nullptr, B, 0ull, (uint64_t)0, (uint64_t)0, (float*)nullptr,
+                     (double*)nullptr, yhat);
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_normalise(float* y, unsigned long long n, double* ms, hipStream_t st) {
-  hipLaunchKernelGGL(k_moments, dim3(1), dim3(256), 0, st, y, n, ms);
+// sums: scratch of 2 kMomentBlocks doubles
+hipError_t launch_mlp_normalise(float* y, unsigned long long n, double* sums, double* ms,
+                                hipStream_t st) {
+  hipLaunchKernelGGL(k_moments_part, dim3(kMomentBlocks), dim3(256), 0, st, y, n, sums);
+  hipLaunchKernelGGL(k_moments, dim3(1), dim3(256), 0, st, sums, n, ms);
   hipLaunchKernelGGL(k_normalise, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, y, n, ms);
   return hipGetLastError();
 }

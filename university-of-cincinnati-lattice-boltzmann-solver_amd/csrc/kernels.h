@@ -223,24 +223,24 @@ struct MlpSamples {               // device-resident training pairs
   unsigned long long* blk = nullptr;      // [blk_n]
   size_t blk_n = 0;
 };
-struct MlpWork {                  // activations of one training batch
-  float *Z1, *A1, *Z2, *A2, *Z3, *A3, *Z4, *A4, *D1, *D2, *D3, *D4;
-  float* part;                    // per-chunk weight-gradient sums: ceil(B / 256) x 4160
+struct MlpWork {                  // of a batch, per block of its kernel (mlp_blocks)
+  float* part;                    // weight-gradient sums, kMlpParams a block
+  double* loss;                   // loss sums
 };
+int mlp_blocks(int B);            // blocks that a batch of B rows takes
 hipError_t launch_mlp_collect(const Box& b, const float* fin, const uint8_t* flags, int stride,
                               int phase, MlpSamples& s, hipStream_t st);
 hipError_t launch_mlp_targets(const double* alpha, MlpSamples& s, unsigned long long first,
                               unsigned long long last, hipStream_t st);
-hipError_t launch_mlp_loss_grad(const float* P, const float* X, const float* y,
-                                const unsigned* idx, int B, MlpWork& w, float* g, double* loss,
-                                hipStream_t st);
-hipError_t launch_mlp_forward_fp32(const float* P, const float* X, int B, MlpWork& w, float* yhat,
+hipError_t launch_mlp_loss_grad(const float* P, const float* X, const float* y, int B,
+                                const MlpWork& w, float* g, double* loss, hipStream_t st);
+hipError_t launch_mlp_train_step(float* P, float* m, float* v, const float* X, const float* y,
+                                 unsigned long long n, uint64_t seed, uint64_t step, int B, int t,
+                                 float lr, const MlpWork& w, double* loss, hipStream_t st);
+hipError_t launch_mlp_forward_fp32(const float* P, const float* X, int B, float* yhat,
                                    hipStream_t st);
-hipError_t launch_mlp_adam(float* P, const float* g, float* m, float* v, int t, float lr,
-                           hipStream_t st);
-hipError_t launch_mlp_gather(const float* X, unsigned long long n, uint64_t seed, uint64_t step,
-                             int B, float* Xb, unsigned* idx, hipStream_t st);
-hipError_t launch_mlp_normalise(float* y, unsigned long long n, double* ms, hipStream_t st);
+hipError_t launch_mlp_normalise(float* y, unsigned long long n, double* sums, double* ms,
+                                hipStream_t st);
 hipError_t launch_mlp_pack(const float* P, short* Wbf, hipStream_t st);
 hipError_t launch_mlp_infer(const float* X, int B, const short* Wbf, const float* P, float* yhat,
                             hipStream_t st);

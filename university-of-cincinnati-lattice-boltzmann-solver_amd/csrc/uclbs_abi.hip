@@ -200,11 +200,11 @@ struct Ctx {
   uclbs::MlpSamples samples;
   bool samples_normalised = false;
   uclbs::MlpWork work{};
-  int work_batch = 0;
-  float* work_buf = nullptr;
-  float* batch_x = nullptr;
-  unsigned* batch_idx = nullptr;
-  double* d_scalar = nullptr;  // loss, mean, std
+  int work_blocks = 0;         // blocks that work_buf serves
+  double* work_buf = nullptr;
+  int stage_rows = 0;          // rows that stage holds: 12 features, 1 target / output
+  float* stage = nullptr;
+  double* d_scalar = nullptr;  // first and last loss, mean, std
   // this device's staging area of uclbs_mlp_forward_noalloc
   float* scratch = nullptr;
   // captured multi-level advance (uclbs_advance with use_graph)
@@ -794,7 +794,7 @@ int uclbs_destroy(void* ctx) {
   for (void* p : {(void*)c->mlp_p, (void*)c->mlp_g, (void*)c->mlp_m, (void*)c->mlp_v,
                   (void*)c->mlp_wbf, (void*)c->samples.X, (void*)c->samples.y,
                   (void*)c->samples.node_of, (void*)c->samples.m_of, (void*)c->samples.count,
-                  (void*)c->samples.ballots, (void*)c->samples.blk, (void*)c->work_buf, (void*)c->batch_x, (void*)c->batch_idx, (void*)c->d_scalar})
+                  (void*)c->samples.ballots, (void*)c->samples.blk, (void*)c->work_buf, (void*)c->stage, (void*)c->d_scalar})
     if (p) (void)hipFree(p);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -2716,26 +2716,31 @@ static int mlp_alloc(Ctx* c) {
 }
 
 static int mlp_work(Ctx* c, int B) {
-  if (c->work_batch >= B) return UCLBS_OK;
-  if (c->work_buf) (void)hipFree(c->work_buf);
-  if (c->batch_x) (void)hipFree(c->batch_x);
-  if (c->batch_idx) (void)hipFree(c->batch_idx);
-  c->work_buf = nullptr;
-  c->batch_x = nullptr;
-  c->batch_idx = nullptr;
-  c->work_batch = 0;
-  const size_t per = (size_t)B * 64;
-  const size_t npart = (size_t)((B + 255) / 256) * (64 * 64 + 64);
-  HIP_TRY(hipMalloc(&c->work_buf, (9 * per + 3 * (size_t)B + npart) * sizeof(float)));
-  float* q = c->work_buf;
-  uclbs::MlpWork& w = c->work;
-  w.Z1 = q; q += per; w.A1 = q; q += per; w.Z2 = q; q += per; w.A2 = q; q += per;
-  w.Z3 = q; q += per; w.A3 = q; q += per; w.D1 = q; q += per; w.D2 = q; q += per;
-  w.D3 = q; q += per; w.Z4 = q; q += B; w.A4 = q; q += B; w.D4 = q; q += B;
-  w.part = q;
-  HIP_TRY(hipMalloc(&c->batch_x, (size_t)B * 12 * sizeof(float)));
-  HIP_TRY(hipMalloc(&c->batch_idx, (size_t)B * sizeof(unsigned)));
-  c->work_batch = B;
+  const int nb = uclbs::mlp_blocks(B);
+  if (c->work_blocks < nb) {
+    if (c->work_buf) (void)hipFree(c->work_buf);
+    c->work_buf = nullptr;
+    c->work_blocks = 0;
+    HIP_TRY(hipMalloc(&c->work_buf,
+                      (size_t)nb * (sizeof(double) + uclbs::kMlpParams * sizeof(float))));
+    c->work_blocks = nb;
+  }
+  c->work.loss = c->work_buf;
+  c->work.part = reinterpret_cast<float*>(c->work_buf + c->work_blocks);
+  return UCLBS_OK;
+}
+
+// device rows of a host batch: B x 12 features at *x, B targets or outputs at *y
+static int mlp_stage_rows(Ctx* c, int B, float** x, float** y) {
+  if (c->stage_rows < B) {
+    if (c->stage) (void)hipFree(c->stage);
+    c->stage = nullptr;
+    c->stage_rows = 0;
+    HIP_TRY(hipMalloc(&c->stage, (size_t)B * 13 * sizeof(float)));
+    c->stage_rows = B;
+  }
+  *x = c->stage;
+  *y = c->stage + (size_t)c->stage_rows * 12;
   return UCLBS_OK;
 }
 
@@ -2800,21 +2805,20 @@ int uclbs_mlp_loss_grad(void* ctx, const float* X, const float* y, int B, float*
   if (!c || !X || !y || !grad || !loss || B <= 0) return set_err(UCLBS_E_ARG, "bad argument");
   if (!c->mlp_p) return set_err(UCLBS_E_STATE, "no network (uclbs_mlp_init)");
   int rc = set_device(c);
-  if (rc || (rc = mlp_work(c, B))) return rc;
   float *dX = nullptr, *dy = nullptr;
-  HIP_TRY(hipMalloc(&dX, (size_t)B * 12 * sizeof(float)));
-  hipError_t e = hipMalloc(&dy, (size_t)B * sizeof(float));
-  if (e == hipSuccess) e = hipMemcpy(dX, X, (size_t)B * 12 * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dy, y, (size_t)B * sizeof(float), hipMemcpyHostToDevice);
+  if (rc || (rc = mlp_work(c, B)) || (rc = mlp_stage_rows(c, B, &dX, &dy))) return rc;
+  hipError_t e = hipMemcpyAsync(dX, X, (size_t)B * 12 * sizeof(float), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
-    e = uclbs::launch_mlp_loss_grad(c->mlp_p, dX, dy, nullptr, B, c->work, c->mlp_g, c->d_scalar,
-                                    c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    e = hipMemcpyAsync(dy, y, (size_t)B * sizeof(float), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
-    e = hipMemcpy(grad, c->mlp_g, uclbs::kMlpParams * sizeof(float), hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(loss, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost);
-  (void)hipFree(dX);
-  if (dy) (void)hipFree(dy);
+    e = uclbs::launch_mlp_loss_grad(c->mlp_p, dX, dy, B, c->work, c->mlp_g, c->d_scalar, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(grad, c->mlp_g, uclbs::kMlpParams * sizeof(float), hipMemcpyDeviceToHost,
+                       c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(loss, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);  // the host arrays are the caller's
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return set_err(UCLBS_E_HIP, "mlp_loss_grad: %s", hipGetErrorString(e));
   return UCLBS_OK;
 }
@@ -2824,18 +2828,16 @@ int uclbs_mlp_forward(void* ctx, const float* X, int B, int use_mfma, float* yha
   if (!c || !X || !yhat || B <= 0) return set_err(UCLBS_E_ARG, "bad argument");
   if (!c->mlp_ready) return set_err(UCLBS_E_STATE, "no network");
   int rc = set_device(c);
-  if (rc || (rc = mlp_work(c, B))) return rc;
   float *dX = nullptr, *dy = nullptr;
-  HIP_TRY(hipMalloc(&dX, (size_t)B * 12 * sizeof(float)));
-  hipError_t e = hipMalloc(&dy, (size_t)B * sizeof(float));
-  if (e == hipSuccess) e = hipMemcpy(dX, X, (size_t)B * 12 * sizeof(float), hipMemcpyHostToDevice);
+  if (rc || (rc = mlp_stage_rows(c, B, &dX, &dy))) return rc;
+  hipError_t e = hipMemcpyAsync(dX, X, (size_t)B * 12 * sizeof(float), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
     e = use_mfma ? uclbs::launch_mlp_infer(dX, B, c->mlp_wbf, c->mlp_p, dy, c->stream)
-                 : uclbs::launch_mlp_forward_fp32(c->mlp_p, dX, B, c->work, dy, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) e = hipMemcpy(yhat, dy, (size_t)B * sizeof(float), hipMemcpyDeviceToHost);
-  (void)hipFree(dX);
-  if (dy) (void)hipFree(dy);
+                 : uclbs::launch_mlp_forward_fp32(c->mlp_p, dX, B, dy, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(yhat, dy, (size_t)B * sizeof(float), hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return set_err(UCLBS_E_HIP, "mlp_forward: %s", hipGetErrorString(e));
   return UCLBS_OK;
 }
@@ -2973,7 +2975,9 @@ int uclbs_mlp_train(void* ctx, int64_t steps, int batch, double lr, uint64_t see
   if ((rc = sample_count(c, &n))) return rc;
   if (n < 2) return set_err(UCLBS_E_STATE, "no training samples (uclbs_mlp_collect)");
   if (!c->samples_normalised) {
-    HIP_TRY(uclbs::launch_mlp_normalise(c->samples.y, n, c->d_scalar + 2, c->stream));
+    HIP_TRY(uclbs::launch_mlp_normalise(c->samples.y, n,
+                                        reinterpret_cast<double*>(c->work.part), c->d_scalar + 2,
+                                        c->stream));
     double ms[2];
     HIP_TRY(hipMemcpyAsync(ms, c->d_scalar + 2, sizeof(ms), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -2984,27 +2988,21 @@ int uclbs_mlp_train(void* ctx, int64_t steps, int batch, double lr, uint64_t see
     c->mlp_ystd = (float)ms[1];
     c->samples_normalised = true;
   }
-  double l0 = 0.0, l1 = 0.0;
   for (int64_t t = 0; t < steps; ++t) {
-    HIP_TRY(uclbs::launch_mlp_gather(c->samples.X, n, seed, (uint64_t)t, batch, c->batch_x,
-                                     c->batch_idx, c->stream));
-    HIP_TRY(uclbs::launch_mlp_loss_grad(c->mlp_p, c->batch_x, c->samples.y, c->batch_idx, batch,
-                                        c->work, c->mlp_g, c->d_scalar, c->stream));
     // learning rate: linear warm-up over the first 2% of the steps, then a
     // cosine decay to 5% of lr (keeps the late steps from undoing the fit)
     const double warm = std::max<double>(1.0, 0.02 * (double)steps);
     const double prog = (double)t / (double)steps;
     const double lrt = t < warm ? lr * (t + 1) / warm
                                 : lr * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(3.141592653589793 * prog)));
-    HIP_TRY(uclbs::launch_mlp_adam(c->mlp_p, c->mlp_g, c->mlp_m, c->mlp_v, ++c->mlp_t, (float)lrt,
-                                   c->stream));
-    if (t == 0 || t == steps - 1) {
-      double l;
-      HIP_TRY(hipMemcpyAsync(&l, c->d_scalar, sizeof(l), hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(hipStreamSynchronize(c->stream));
-      (t == 0 ? l0 : l1) = l;
-    }
+    HIP_TRY(uclbs::launch_mlp_train_step(c->mlp_p, c->mlp_m, c->mlp_v, c->samples.X, c->samples.y,
+                                         n, seed, (uint64_t)t, batch, ++c->mlp_t, (float)lrt,
+                                         c->work, c->d_scalar + (t == 0 ? 0 : 1), c->stream));
   }
+  double l01[2];
+  HIP_TRY(hipMemcpyAsync(l01, c->d_scalar, sizeof(l01), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  const double l0 = l01[0], l1 = l01[1];
   if (loss_first) *loss_first = l0;
   if (loss_last) *loss_last = steps == 1 ? l0 : l1;
   if (!std::isfinite(l0) || !std::isfinite(steps == 1 ? l0 : l1))
