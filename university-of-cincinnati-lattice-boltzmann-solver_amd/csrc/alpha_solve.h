@@ -47,9 +47,13 @@ constexpr double kTrivialX = 1e-12;
 // (1e-16 in FP64 mode, i.e. exact to round-off; tol / 2 in FP32 mode, so
 // truncation adds at most half the Newton tolerance to the residual of g).
 struct SeriesThr {
-  double m5, m7, m10, m16;  // general path orders
+  double m7, m10, m16;      // FP64 storage: orders 7, 10, 16
   float m_fast;             // order kFastOrder of the fused FP32-storage pass
   float m_mid;              // order kMidOrder, the second in-register tier
+};
+template <int N>
+struct Order {
+  static constexpr int value = N;
 };
 constexpr int kFastOrder = 6;
 constexpr int kMidOrder = 12;
@@ -57,44 +61,8 @@ inline double series_limit(int N, double eps) {
   return __builtin_pow(eps * N * (N - 1.0), 1.0 / (N - 1.0)) / 2.2;
 }
 inline SeriesThr make_series_thr(double eps) {
-  return SeriesThr{series_limit(5, eps), series_limit(7, eps), series_limit(10, eps),
-                   series_limit(16, eps), (float)series_limit(kFastOrder, eps),
+  return SeriesThr{series_limit(7, eps), series_limit(10, eps), series_limit(16, eps), (float)series_limit(kFastOrder, eps),
                    (float)series_limit(kMidOrder, eps)};
-}
-
-// ln(1 + x) for x > -1 in FP64, about 35 VALU operations: u = 1 + x = 2^e m
-// with m in [sqrt(1/2), sqrt(2)), ln m = 2 atanh(s), s = (m-1)/(m+1), |s| <=
-// 0.1716, summed to s^23 (remainder < 1e-18); ln 2 split in a high part exact
-// in e*ln2_hi and a low part; the rounding error of 1 + x is removed to first
-// order, ln(1+x) = ln(u) - ((u - 1) - x)/u.
-__host__ __device__ __forceinline__ double log1p_fast(double x) {
-  const double u = 1.0 + x;
-  const double c = (u - 1.0) - x;
-  int e;
-  double m = __builtin_frexp(u, &e);  // u = m 2^e, m in [0.5, 1)
-  if (m < 0.70710678118654752440) {
-    m *= 2.0;
-    e -= 1;
-  }
-  const double s = (m - 1.0) / (m + 1.0);
-  const double s2 = s * s;
-  // 2 * sum_{k=0..11} s2^k / (2k+1)
-  double p = 2.0 / 23.0;
-  p = p * s2 + 2.0 / 21.0;
-  p = p * s2 + 2.0 / 19.0;
-  p = p * s2 + 2.0 / 17.0;
-  p = p * s2 + 2.0 / 15.0;
-  p = p * s2 + 2.0 / 13.0;
-  p = p * s2 + 2.0 / 11.0;
-  p = p * s2 + 2.0 / 9.0;
-  p = p * s2 + 2.0 / 7.0;
-  p = p * s2 + 2.0 / 5.0;
-  p = p * s2 + 2.0 / 3.0;
-  p = p * s2 + 2.0;
-  const double ln2_hi = 6.93147180369123816490e-01;  // 0x3FE62E42FEE00000, 32 significant bits
-  const double ln2_lo = 1.90821492927058770002e-10;
-  const double de = (double)e;
-  return de * ln2_hi + (de * ln2_lo + s * p) - c / u;
 }
 
 // 1/v for a normal v: the hardware estimate and two Newton steps (each at
@@ -106,9 +74,13 @@ __device__ __forceinline__ double drcp(double v) {
   return r;
 }
 
-// log1p_fast with both divisions replaced by reciprocals (device only): the
-// quotient s only needs relative accuracy (its error enters ln as 2 ds with
-// |s| <= 0.1716), and c/u is a first-order correction of size eps
+// ln(1 + x) for x > -1 in FP64, about 30 VALU operations: u = 1 + x = 2^e m
+// with m in [sqrt(1/2), sqrt(2)), ln m = 2 atanh(s), s = (m-1)/(m+1), |s| <=
+// 0.1716, summed to s^23 (remainder < 1e-18); ln 2 split in a high part exact
+// in e*ln2_hi and a low part; the rounding error of 1 + x is removed to first
+// order, ln(1+x) = ln(u) - ((u - 1) - x)/u.  Reciprocals for both quotients: s
+// only needs relative accuracy (its error enters ln as 2 ds), and c/u is a
+// correction of size eps.
 __device__ __forceinline__ double log1p_dev(double x) {
   const double u = 1.0 + x;
   const double c = (u - 1.0) - x;
@@ -132,7 +104,7 @@ __device__ __forceinline__ double log1p_dev(double x) {
   p = p * s2 + 2.0 / 5.0;
   p = p * s2 + 2.0 / 3.0;
   p = p * s2 + 2.0;
-  const double ln2_hi = 6.93147180369123816490e-01;
+  const double ln2_hi = 6.93147180369123816490e-01;  // 0x3FE62E42FEE00000, 32 significant bits
   const double ln2_lo = 1.90821492927058770002e-10;
   const double de = (double)e;
   return de * ln2_hi + (de * ln2_lo + s * p) - c * __builtin_amdgcn_rcp(u);
@@ -176,54 +148,36 @@ __device__ __forceinline__ double log1p_tab(double y, const LogTable& t) {
   return (de * ln2_hi + t.L[k]) + (de * ln2_lo + p * r);
 }
 
-// phi(y) = (1 + y) ln(1 + y) - y, series for small |y|, direct otherwise
-__device__ __forceinline__ double phi1p(double y) {
-  if (fabs(y) < 0.1) {
-    double s = 0.0, p = y * y;
+// The series as a polynomial: with C_n = (-1)^n S_n / (n (n-1)) and
+// L = sum (-1)^n S_n / (n-1),
+//     g(a) = a^2 Q(a) - L a,  g'(a) = a (2 Q(a) + a Q'(a)) - L,  Q = sum C_n a^(n-2),
+// so that an evaluation is two FMAs an order (Horner and its derivative) and
+// the coefficient's product where the terms one by one take six operations an
+// order.  sn(n) yields S_n; the coefficients are formed as they are used, since
+// keeping them (2 N registers) would cost the FP32 kernels their occupancy.
+template <int N, class SN>
+struct SeriesPoly {
+  SN sn;
+  double L;
+  __device__ __forceinline__ explicit SeriesPoly(SN s) : sn(s), L(0.0) {
 #pragma unroll
-    for (int n = 2; n <= 20; ++n) {
-      s += ((n & 1) ? -p : p) * (1.0 / (n * (n - 1.0)));
-      p *= y;
+    for (int n = N; n >= 2; --n) L = fma(sn(n), ((n & 1) ? -1.0 : 1.0) / (n - 1.0), L);
+  }
+  __device__ __forceinline__ void operator()(double a, double& g, double& gp) const {
+    double q = sn(N) * (((N & 1) ? -1.0 : 1.0) / (N * (N - 1.0))), dq = 0.0;
+#pragma unroll
+    for (int n = N - 1; n >= 2; --n) {
+      dq = fma(dq, a, q);
+      q = fma(q, a, sn(n) * (((n & 1) ? -1.0 : 1.0) / (n * (n - 1.0))));
     }
-    return s;
+    const double aq = a * q;
+    g = a * (aq - L);
+    gp = fma(a, fma(a, dq, q + q), -L);
   }
-  return (1.0 + y) * log1p(y) - y;
-}
-
-template <int N>
-__device__ __forceinline__ void series_g(const double* S, double a, double& g, double& gp) {
-  double an1 = a, sg = 0.0, sgp = 0.0;
-#pragma unroll
-  for (int n = 2; n <= N; ++n) {
-    const double an = an1 * a;
-    const double c1 = 1.0 / (n * (n - 1.0)), c2 = 1.0 / (n - 1.0);
-    const double tg = S[n] * (an * c1 - a * c2);
-    const double tgp = S[n] * ((an1 - 1.0) * c2);
-    if (n & 1) { sg -= tg; sgp -= tgp; } else { sg += tg; sgp += tgp; }
-    an1 = an;
-  }
-  g = sg;
-  gp = sgp;
-}
-
-// Same series with the orders split over two arrays: S[2..N1] and Sh[0..N2-N1-1]
-// holding orders N1+1..N2 (keeps the second tier's registers small).
-template <int N1, int N2>
-__device__ __forceinline__ void series_g2(const double* S, const double* Sh, double a, double& g,
-                                          double& gp) {
-  double an1 = a, sg = 0.0, sgp = 0.0;
-#pragma unroll
-  for (int n = 2; n <= N2; ++n) {
-    const double an = an1 * a;
-    const double c1 = 1.0 / (n * (n - 1.0)), c2 = 1.0 / (n - 1.0);
-    const double Sn = n <= N1 ? S[n] : Sh[n - N1 - 1];
-    const double tg = Sn * (an * c1 - a * c2);
-    const double tgp = Sn * ((an1 - 1.0) * c2);
-    if (n & 1) { sg -= tg; sgp -= tgp; } else { sg += tg; sgp += tgp; }
-    an1 = an;
-  }
-  g = sg;
-  gp = sgp;
+};
+template <int N, class SN>
+__device__ __forceinline__ SeriesPoly<N, SN> series_poly(SN sn) {
+  return SeriesPoly<N, SN>(sn);
 }
 
 // Safeguarded Newton shared by both evaluations of g.  Iterations count Newton
@@ -243,7 +197,8 @@ __device__ __forceinline__ AlphaOut newton_alpha(Eval&& ev, double S2, double am
     if (g < 0.0 && a >= amax) { r.alpha = amax; r.iters = k; r.status = ALPHA_BOUND; return r; }
     if (k >= maxit) { r.alpha = a; r.iters = k; r.status = ALPHA_NOCONV; return r; }
     if (g < 0.0) lo = a; else { hi = a; hi_is_bound = false; }
-    double an = a - g / gp;
+    // (a zero or infinite g' gives NaN: the middle of the bracket)
+    double an = fma(-g, drcp(gp), a);
     if (!(an > lo && an < hi)) an = (hi_is_bound && an >= hi) ? amax : 0.5 * (lo + hi);
     if (an == amax) hi_is_bound = false;
     a = an;
@@ -370,79 +325,79 @@ __device__ __forceinline__ AlphaOut recentred_alpha(DX&& dx, FX&& fx, LG&& lg, d
   }
 }
 
-template <int N, class XF>
-__device__ __forceinline__ void power_sums(XF&& dx, int q, double* S) {
+// S_2..S_N of f x^n = D x^(n-1) over the 27 directions: two orders share a
+// product, D x^(2k) times x and times x^2
+template <int N>
+__device__ __forceinline__ void power_sums27(const double (&D)[27], const double (&x)[27],
+                                             double (&S)[N + 1]) {
 #pragma unroll
   for (int n = 2; n <= N; ++n) S[n] = 0.0;
 #pragma unroll
-  for (int i = 0; i < q; ++i) {
-    double d, x;
-    dx(i, d, x);
-    double t = d * x;  // f x^2
-    S[2] += t;
+  for (int i = 0; i < 27; ++i) {
+    const double y = x[i] * x[i];
+    double t = D[i];
 #pragma unroll
-    for (int n = 3; n <= N; ++n) { t *= x; S[n] += t; }
+    for (int n = 2; n <= N; n += 2) {
+      S[n] = fma(t, x[i], S[n]);
+      if (n < N) S[n + 1] = fma(t, y, S[n + 1]);
+      if (n + 2 <= N) t *= y;
+    }
   }
 }
 
-// dx(i, d, x) yields D_i and x_i in FP64; fx(i) yields f_i in FP64.
-template <int Q, class DX, class FX>
-__device__ AlphaOut solve_alpha(DX&& dx, FX&& fx, double m, double xmin, double S2,
-                                double alpha0, double tol, int maxit, const SeriesThr& thr) {
+// alpha of an FP64 node from D_i, x_i = D_i / f_i, m = max|x|, xmin = min x.
+// The order of the series is the wavefront's (its largest m decides), so that
+// its lanes run one Newton; a lane beyond order 16 takes direct logarithms.
+__device__ __forceinline__ AlphaOut solve_alpha27(const double (&f)[27], const double (&D)[27],
+                                                  const double (&x)[27], bool nonpos, double m,
+                                                  double xmin, double alpha0, double tol, int maxit,
+                                                  const SeriesThr& thr) {
   const double amax = xmin < 0.0 ? -1.0 / xmin : 1e300;
-  if (m < kTrivialX) return AlphaOut{2.0, 0, ALPHA_TRIVIAL, false};
-  if (amax < 2.0) return AlphaOut{amax, 0, ALPHA_BOUND, false};
-  double S[17];
-  if (m <= thr.m7) {
-    if (m <= thr.m5) {
-      power_sums<5>(dx, Q, S);
-      return newton_alpha([&](double a, double& g, double& gp) __attribute__((always_inline)) { series_g<5>(S, a, g, gp); },
-                          S2, amax, alpha0, tol, maxit);
+  AlphaOut r{2.0, 0, ALPHA_TRIVIAL, false};
+  bool open = false;
+  if (nonpos) r.status = ALPHA_NONPOS;
+  else if (m < kTrivialX) r.status = ALPHA_TRIVIAL;
+  else if (amax < 2.0) r = AlphaOut{amax, 0, ALPHA_BOUND, false};
+  else open = true;
+  auto series = [&](auto order) __attribute__((always_inline)) {
+    constexpr int N = decltype(order)::value;
+    double S[N + 1];
+    power_sums27<N>(D, x, S);
+    const auto ev = series_poly<N>([&](int n) __attribute__((always_inline)) { return S[n]; });
+    if (open && m <= thr.m16) r = newton_alpha(ev, S[2], amax, alpha0, tol, maxit);
+  };
+  const bool wide = open && m > thr.m7 && m <= thr.m16;
+  if (__any(wide && m > thr.m10)) series(Order<16>());
+  else if (__any(wide)) series(Order<10>());
+  else if (__any(open && m <= thr.m16)) series(Order<7>());
+  if (open && !(m <= thr.m16)) {
+    // g(a) = sum f ((1 + y) ln(1 + y) - y) - a K, y = a x, K = sum D ln(1 + x);
+    // (1+y) ln(1+y) - y loses only absolute accuracy O(eps |y|), far below
+    // tol * S2
+    double K = 0.0, S2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < 27; ++i) {
+      K = fma(D[i], log1p_dev(x[i]), K);
+      S2 = fma(D[i], x[i], S2);
     }
-    power_sums<7>(dx, Q, S);
-    return newton_alpha([&](double a, double& g, double& gp) __attribute__((always_inline)) { series_g<7>(S, a, g, gp); }, S2,
-                        amax, alpha0, tol, maxit);
-  }
-  if (m <= thr.m10) {
-    power_sums<10>(dx, Q, S);
-    return newton_alpha([&](double a, double& g, double& gp) __attribute__((always_inline)) { series_g<10>(S, a, g, gp); },
-                        S2, amax, alpha0, tol, maxit);
-  }
-  if (m <= thr.m16) {
-    power_sums<16>(dx, Q, S);
-    return newton_alpha([&](double a, double& g, double& gp) __attribute__((always_inline)) { series_g<16>(S, a, g, gp); },
-                        S2, amax, alpha0, tol, maxit);
-  }
-  // large non-equilibrium: direct logarithms, x_i and ln(1 + x_i) formed once
-  // (with log1p_fast each evaluation costs 27 logarithms of ~35 operations)
-  double xs[Q], l1[Q];
+    r = newton_alpha(
+        [&](double a, double& g, double& gp) __attribute__((always_inline)) {
+          double sg = 0.0, sgp = 0.0;
+          bool inf_gp = false;
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    double d;
-    dx(i, d, xs[i]);
-    l1[i] = log1p_fast(xs[i]);
+          for (int i = 0; i < 27; ++i) {
+            const double y = a * x[i], u = 1.0 + y;
+            if (u <= 0.0) { sg -= f[i] * y; inf_gp = true; continue; }  // limit of u ln u at 0
+            const double la = log1p_dev(y);
+            sg = fma(f[i], fma(u, la, -y), sg);
+            sgp = fma(D[i], la, sgp);
+          }
+          g = fma(-a, K, sg);
+          gp = inf_gp ? __builtin_huge_val() : sgp - K;
+        },
+        S2, amax, alpha0, tol, maxit);
+    r.logpath = true;
   }
-  AlphaOut r = newton_alpha(
-      [&](double a, double& g, double& gp) __attribute__((always_inline)) {
-        double sg = 0.0, sgp = 0.0;
-        bool inf_gp = false;
-#pragma unroll
-        for (int i = 0; i < Q; ++i) {
-          const double x = xs[i];
-          const double f = fx(i);
-          const double y = a * x;
-          if (1.0 + y <= 0.0) { sg += f * (-y - y * l1[i]); inf_gp = true; continue; }
-          const double la = log1p_fast(y);
-          // (1+y) ln(1+y) - y loses only absolute accuracy O(eps*|y|), far
-          // below tol * S2
-          sg += f * ((1.0 + y) * la - y - y * l1[i]);
-          sgp += f * x * (la - l1[i]);
-        }
-        g = sg;
-        gp = inf_gp ? __builtin_huge_val() : sgp;
-      },
-      S2, amax, alpha0, tol, maxit);
-  r.logpath = true;
   return r;
 }
 

@@ -161,9 +161,7 @@ __device__ __forceinline__ AlphaOut collide27_shifted(float (&f)[27], double bet
       ao = AlphaOut{amax, 0, ALPHA_BOUND, false};
     } else if (!__any(m > ac.thr.m_fast)) {
       // the whole wavefront is within the fused order: Newton on the scalar series
-      auto ev = [&](double a, double& g, double& gp) __attribute__((always_inline)) {
-        series_g<kFastOrder>(S, a, g, gp);
-      };
+      const auto ev = series_poly<kFastOrder>([&](int n) __attribute__((always_inline)) { return S[n]; });
       if (ac.mode == 2) {
         // learned start; the plain start takes over when it is outside the
         // bracket or does not converge
@@ -194,18 +192,19 @@ __device__ __forceinline__ AlphaOut collide27_shifted(float (&f)[27], double bet
 #pragma unroll
         for (int q = 0; q < kMidOrder - kFastOrder; ++q) { t *= x; Sh[q] += t; }
       }
-      double Shd[kMidOrder > kFastOrder ? kMidOrder - kFastOrder : 1];
-#pragma unroll
-      for (int q = 0; q < kMidOrder - kFastOrder; ++q) Shd[q] = (double)Sh[q];
+      const auto ev = series_poly<kMidOrder>([&](int n) __attribute__((always_inline)) {
+        if (n <= kFastOrder) return S[n];
+        // converted anew on each use: hoisted out of the Newton loop, the
+        // products of the sums would spill
+        float c = Sh[n - kFastOrder - 1];
+        __asm__ volatile("" : "+v"(c));
+        return (double)c;
+      });
       // one Newton for both kinds of lane: to the tolerance within the tier,
       // to a seed (1e-6, at most 8 updates) for a lane beyond it
       const bool far = m > ac.thr.m_mid;
       const double a0 = ac.mode == 2 ? alpha0 : 2.0;
-      ao = newton_alpha(
-          [&](double a, double& g, double& gp) __attribute__((always_inline)) {
-            series_g2<kFastOrder, kMidOrder>(S, Shd, a, g, gp);
-          },
-          S[2], amax, a0, far ? 1e-6 : ac.tol, far ? 8 : ac.maxit);
+      ao = newton_alpha(ev, S[2], amax, a0, far ? 1e-6 : ac.tol, far ? 8 : ac.maxit);
       if (far) return AlphaOut{ao.alpha, ao.iters, ALPHA_DEFER, false};
     }
   }
@@ -278,6 +277,9 @@ __device__ __forceinline__ AlphaOut collide27_far(float (&f)[27], double beta, c
 }
 
 // ---------------------------------------------------------------- FP64 full
+// f, D and x = D / f of the node stay in registers (162 VGPRs of the 256 that
+// two wavefronts a SIMD leave each), reciprocals replace the quotients, and
+// the sums and logarithms read x instead of dividing again.
 __device__ __forceinline__ AlphaOut collide27_fp64(double (&f)[27], double beta,
                                                    const AlphaCfg& ac, double alpha0,
                                                    double& rho_out, double (&u_out)[3]) {
@@ -289,45 +291,46 @@ __device__ __forceinline__ AlphaOut collide27_fp64(double (&f)[27], double beta,
     if (CY27[i] > 0) jy += f[i]; else if (CY27[i] < 0) jy -= f[i];
     if (CZ27[i] > 0) jz += f[i]; else if (CZ27[i] < 0) jz -= f[i];
   }
-  const double ux = jx / r, uy = jy / r, uz = jz / r;
+  const double inv = drcp(r);
+  const double ux = jx * inv, uy = jy * inv, uz = jz * inv;
   rho_out = r;
   u_out[0] = ux; u_out[1] = uy; u_out[2] = uz;
   // 1-D factors in the oracle's direct form
-  double px[3], py[3], pz[3];
-  auto psi = [](double u, double* p) {
+  double px[3], pyz[9];
+  auto psi = [](double u, double* p) __attribute__((always_inline)) {
     const double s = sqrt(1.0 + 3.0 * u * u);
-    const double b = 2.0 - s;
+    const double b = 2.0 - s, v = 1.0 - u, w = 2.0 * u + s;
+    const double q = drcp(v * w);
     p[1] = b;
-    p[2] = b * (2.0 * u + s) / (1.0 - u);
-    p[0] = b * (1.0 - u) / (2.0 * u + s);
+    p[2] = b * (w * w) * q;
+    p[0] = b * (v * v) * q;
   };
-  psi(ux, px); psi(uy, py); psi(uz, pz);
-  double D[27];
-  double m = 0.0, xmin = 0.0, S2 = 0.0;
-  bool nonpos = false;
+  {
+    double py[3], pz[3];
+    psi(ux, px); psi(uy, py); psi(uz, pz);
 #pragma unroll
-  for (int i = 0; i < 27; ++i) {
-    const double feq = r * W27[i] * px[CX27[i] + 1] * py[CY27[i] + 1] * pz[CZ27[i] + 1];
-    D[i] = feq - f[i];
+    for (int c = 0; c < 3; ++c) px[c] *= r;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) pyz[c] = py[c / 3] * pz[c % 3];
   }
+  double D[27];
+#pragma unroll
+  for (int i = 0; i < 27; ++i)
+    D[i] = fma(W27[i] * px[CX27[i] + 1], pyz[(CY27[i] + 1) * 3 + CZ27[i] + 1], -f[i]);
   AlphaOut ao{2.0, 0, ALPHA_TRIVIAL, false};
   if (ac.mode != 1) {
+    double x[27];
+    double m = 0.0, xmin = 0.0;
+    bool nonpos = false;
 #pragma unroll
     for (int i = 0; i < 27; ++i) {
       nonpos |= !(f[i] > 0.0);
-      const double x = D[i] / f[i];
-      m = fmax(m, fabs(x));
-      xmin = fmin(xmin, x);
-      S2 += D[i] * x;
+      x[i] = D[i] * drcp(f[i]);
+      m = fmax(m, fabs(x[i]));
+      xmin = fmin(xmin, x[i]);
     }
-    if (nonpos) {
-      ao = AlphaOut{2.0, 0, ALPHA_NONPOS, false};
-    } else {
-      auto dx = [&](int i, double& d, double& x) __attribute__((always_inline)) { d = D[i]; x = D[i] / f[i]; };
-      auto fx = [&](int i) __attribute__((always_inline)) { return f[i]; };
-      ao = solve_alpha<27>(dx, fx, m, xmin, S2, ac.mode == 2 ? alpha0 : 2.0, ac.tol, ac.maxit,
-                           ac.thr);
-    }
+    ao = solve_alpha27(f, D, x, nonpos, m, xmin, ac.mode == 2 ? alpha0 : 2.0, ac.tol, ac.maxit,
+                       ac.thr);
   }
   const double ab = ao.alpha * beta;
 #pragma unroll

@@ -101,7 +101,7 @@ __device__ __forceinline__ void queue_far(const StepArgs& a, unsigned shard, boo
 // kFlags: the level has link tables; only interior fluid nodes (flag 0) are
 // updated here, the boundary kernel updates the rest.
 template <bool kShifted, bool kKeepAlpha, bool kFlags>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k27_step_periodic(const void* __restrict__ fin_,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 4 : 2))) void k27_step_periodic(const void* __restrict__ fin_,
                                                          void* __restrict__ fout_,
                                                          double* __restrict__ alpha_out,
                                                          unsigned long long* __restrict__ stats,
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // kernel like s).  Ghosts at a coarse-fine interface are interpolated before
 // the step.
 template <bool kShifted, bool kKeepAlpha, bool kLinks>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k27_step_boxes(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 4 : 2))) void k27_step_boxes(
     const void* __restrict__ fin_, void* __restrict__ fout_, double* __restrict__ alpha_out,
     unsigned long long* __restrict__ stats, unsigned nn, StepArgs a,
     const uint8_t* __restrict__ flags, const uint4* __restrict__ alias,
