@@ -476,6 +476,20 @@ __global__ void k27_init_tgv(void* __restrict__ dst_, Box dom, int64_t nn, int64
 }
 
 
+__device__ void feq27_fp64(double rho, const double u[3], double* feq) {
+  double p[3][3];
+  for (int d = 0; d < 3; ++d) {
+    const double s = sqrt(1.0 + 3.0 * u[d] * u[d]);
+    const double bb = 2.0 - s;
+    p[d][1] = bb;
+    p[d][2] = bb * (2.0 * u[d] + s) / (1.0 - u[d]);
+    p[d][0] = bb * (1.0 - u[d]) / (2.0 * u[d] + s);
+  }
+#pragma unroll
+  for (int i = 0; i < 27; ++i)
+    feq[i] = rho * W27[i] * p[0][CX27[i] + 1] * p[1][CY27[i] + 1] * p[2][CZ27[i] + 1];
+}
+
 // ------------------------------------------------------------------ boundaries
 // One thread per fluid node that has a boundary link.  The incoming population
 // f_i(x) (velocity c_i, from x - c_i) is chosen by the code s of the link from
@@ -498,129 +512,122 @@ __global__ void k27_init_tgv(void* __restrict__ dst_, Box dom, int64_t nn, int64
 //                  are convex combinations, so no population turns negative)
 //   other          fout_opp(i)(x)
 // The node then collides with the streaming kernel's collide.  All BC
-// arithmetic is FP64.
+// arithmetic is FP64; opposite directions have the same weight and the two
+// factors of an interpolated link add to one, so that it is formed on the
+// stored deviations f - w as on full populations.
+//
+// The list is short (the cells around a body: a few wavefronts a CU at most),
+// so one node's chain of memory waits bounds the kernel.  The chain is four
+// long: list, all 26 link codes, one population a direction, the second
+// population of the wall links; a loop over the wall links that read code,
+// populations and the node behind one after the other took 102 us on the
+// 149 x 77 x 61 duct.
 template <bool kShifted>
-__device__ __forceinline__ double ldf(const void* f, int i, int64_t n, int64_t k) {
-  if constexpr (kShifted) return W27[i] + (double)static_cast<const float*>(f)[(int64_t)i * n + k];
-  else return static_cast<const double*>(f)[(int64_t)i * n + k];
-}
-
-__device__ __forceinline__ int wrapc(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
-
-__device__ void feq27_fp64(double rho, const double u[3], double* feq) {
-  double p[3][3];
-  for (int d = 0; d < 3; ++d) {
-    const double s = sqrt(1.0 + 3.0 * u[d] * u[d]);
-    const double bb = 2.0 - s;
-    p[d][1] = bb;
-    p[d][2] = bb * (2.0 * u[d] + s) / (1.0 - u[d]);
-    p[d][0] = bb * (1.0 - u[d]) / (2.0 * u[d] + s);
-  }
-#pragma unroll
-  for (int i = 0; i < 27; ++i)
-    feq[i] = rho * W27[i] * p[0][CX27[i] + 1] * p[1][CY27[i] + 1] * p[2][CZ27[i] + 1];
-}
-
-template <bool kShifted>
-__global__ __launch_bounds__(64) void k27_boundary(const void* __restrict__ fin,
+__global__ __launch_bounds__(64) void k27_boundary(const void* __restrict__ fin_,
                                                     void* __restrict__ fout_,
                                                     double* __restrict__ alpha, int keep_alpha,
                                                     unsigned long long* __restrict__ stats,
                                                     Box b, StepArgs a, BcArgs bc) {
+  using T = typename std::conditional<kShifted, float, double>::type;
+  const T* __restrict__ fin = static_cast<const T*>(fin_);
+  T* __restrict__ fout = static_cast<T*>(fout_);
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = j < bc.nlist;
-  const int64_t k = bc.list[active ? j : 0];
-  const int64_t n = b.n;
+  const unsigned k = bc.list[active ? j : 0];
+  const unsigned nn = (unsigned)b.n;
   // the node's box: the level's one box (periodic axes wrap) or, on a level
   // of many boxes, the box whose ghost shell holds the node's neighbours
-  int64_t base = 0;
-  int bnx = b.nx, bny = b.ny, bnz = b.nz;
+  unsigned base = 0, nx = (unsigned)b.nx, ny = (unsigned)b.ny, nz = (unsigned)b.nz;
   if (bc.boxes) {
     const BoxDesc bx = bc.boxes[bc.box_of[active ? j : 0]];
-    base = bx.off;
-    bnx = (int)bx.nx;
-    bny = (int)bx.ny;
-    bnz = (int)(bx.n / (bx.nx * bx.ny));
+    base = (unsigned)bx.off;
+    nx = bx.nx;
+    ny = bx.ny;
+    nz = (unsigned)(bx.n / (bx.nx * bx.ny));
   }
-  const int64_t lk = k - base;
-  const int x = (int)(lk % bnx);
-  const int64_t yz = lk / bnx;
-  const int y = (int)(yz % bny), z = (int)(yz / bny);
-  double f[27];
-  bool unknown[27];
-  bool any_wall = false;
+  int32_t s[27];  // code of the link towards x - c_i
 #pragma unroll
-  for (int i = 0; i < 27; ++i) {
-    unknown[i] = false;
-    if (i == 0) { f[0] = ldf<kShifted>(fin, 0, n, k); continue; }
-    const int32_t s = bc.state[(int64_t)OPP27[i] * n + k];
-    if (s >= 0) {
-      const int64_t src = base + wrapc(x - CX27[i], bnx) +
-                          (int64_t)bnx * (wrapc(y - CY27[i], bny) + (int64_t)bny * wrapc(z - CZ27[i], bnz));
-      f[i] = ldf<kShifted>(fin, i, n, src);
-    } else if (s == -10) {
-      f[i] = ldf<kShifted>(fin, OPP27[i], n, k);
-    } else if (s <= -100 && s >= -199 && -s - 100 <= bc.n_in) {
-      f[i] = bc.feq_in[(int64_t)(-s - 101) * 27 + i];
-    } else if (s <= -200 && s >= -299 && -s - 200 <= bc.n_out) {
-      f[i] = bc.feq_out[(int64_t)(-s - 201) * 27 + i];
-    } else if (s == -1000 && bc.feq_fs) {
-      f[i] = bc.feq_fs[i];
-    } else if (s <= -1001) {
-      unknown[i] = true;
-      any_wall = true;
-      f[i] = 0.0;
-    } else {
-      f[i] = ldf<kShifted>(fin, OPP27[i], n, k);
-    }
+  for (int i = 1; i < 27; ++i) s[i] = (bc.state + (size_t)OPP27[i] * nn)[k];
+  const unsigned lk = k - base, x = lk % nx, yz = lk / nx, y = yz % ny, z = yz / ny;
+  // node x - c, c = -1, 0, +1 along each axis (wrapped)
+  unsigned ox[3], oy[3], oz[3];
+  ox[0] = x + 1 == nx ? 0u : x + 1;
+  ox[1] = x;
+  ox[2] = x == 0 ? nx - 1 : x - 1;
+  oy[0] = (y + 1 == ny ? 0u : y + 1) * nx;
+  oy[1] = y * nx;
+  oy[2] = (y == 0 ? ny - 1 : y - 1) * nx;
+  oz[0] = base + (z + 1 == nz ? 0u : z + 1) * nx * ny;
+  oz[1] = base + z * nx * ny;
+  oz[2] = base + (z == 0 ? nz - 1 : z - 1) * nx * ny;
+  auto from = [&](int i) __attribute__((always_inline)) {
+    return ox[CX27[i] + 1] + oy[CY27[i] + 1] + oz[CZ27[i] + 1];
+  };
+  // the pulled population, or the node's own opposite one (bounce-back, the
+  // first value of a wall link, and any other code)
+  T f[27];
+  f[0] = fin[k];
+  bool tables = false, walls = false;
+#pragma unroll
+  for (int i = 1; i < 27; ++i) {
+    const bool pull = s[i] >= 0;
+    const T* p = pull ? fin + (size_t)i * nn : fin + (size_t)OPP27[i] * nn;
+    f[i] = p[pull ? from(i) : k];
+    tables |= s[i] <= -101 && s[i] >= -1000;
+    walls |= s[i] <= -1001;
   }
   int nibb = 0;
-  if (any_wall && active) {
-#pragma unroll 1
+  if (walls) {
+    // the second population of an interpolated link: q >= 1/2 the node's own
+    // f_i, else the opposite one of the fluid node behind, x + c_i
+    T w[27];
+#pragma unroll
     for (int i = 1; i < 27; ++i) {
-      if (!unknown[i]) continue;
-      const int kk = OPP27[i];
-      const double q = fabs((double)bc.state[(int64_t)kk * n + k] + 1001.0) / 1.0e9;
-      const double fk = ldf<kShifted>(fin, kk, n, k);
-      double v;
-      if (q >= 0.5) {
-        v = fk / (2.0 * q) + (1.0 - 1.0 / (2.0 * q)) * ldf<kShifted>(fin, i, n, k);
-      } else if (bc.state[(int64_t)i * n + k] >= 0) {
-        // the fluid node behind x, x + c_i
-        const int64_t src = base + wrapc(x + CX27[i], bnx) +
-                            (int64_t)bnx * (wrapc(y + CY27[i], bny) + (int64_t)bny * wrapc(z + CZ27[i], bnz));
-        v = 2.0 * q * fk + (1.0 - 2.0 * q) * ldf<kShifted>(fin, kk, n, src);
-      } else {
-        v = fk;
+      w[i] = f[i];
+      if (s[i] <= -1001) {
+        const bool far = -(s[i] + 1001) >= 500000000;
+        if (far || s[OPP27[i]] >= 0) {
+          const T* p = far ? fin + (size_t)i * nn : fin + (size_t)OPP27[i] * nn;
+          w[i] = p[far ? k : from(OPP27[i])];
+        }
       }
-      f[i] = v;
-      nibb++;
+    }
+#pragma unroll
+    for (int i = 1; i < 27; ++i)
+      if (s[i] <= -1001) {
+        const int q9 = -(s[i] + 1001);
+        const double q2 = (double)q9 * 2e-9;
+        const double c = q9 >= 500000000 ? drcp(q2) : q2;
+        f[i] = (T)fma(c, (double)f[i] - (double)w[i], (double)w[i]);
+        nibb++;
+      }
+  }
+  if (tables) {
+#pragma unroll
+    for (int i = 1; i < 27; ++i) {
+      const double* tab = s[i] <= -101 && s[i] >= -199 && -s[i] - 100 <= bc.n_in
+                              ? bc.feq_in + (size_t)(-s[i] - 101) * 27
+                          : s[i] <= -201 && s[i] >= -299 && -s[i] - 200 <= bc.n_out
+                              ? bc.feq_out + (size_t)(-s[i] - 201) * 27
+                          : s[i] == -1000 ? bc.feq_fs
+                                          : nullptr;
+      if (tab) f[i] = (T)(kShifted ? tab[i] - W27[i] : tab[i]);
     }
   }
   AlphaCfg ac{a.tol, a.maxit, a.alpha_mode, a.thr};
   double rho, u[3];
   AlphaOut ao;
-  if constexpr (kShifted) {
-    // the streaming kernel's collide: a node beyond the series tiers stores
-    // its pre-collision state and joins the far-from-equilibrium queue
-    float fs[27];
+  // the streaming kernel's collide: a node beyond the series tiers stores its
+  // pre-collision state and joins the far-from-equilibrium queue
+  if constexpr (kShifted) ao = collide27_shifted(f, a.beta, ac, 2.0, rho, u);
+  else ao = collide27_fp64(f, a.beta, ac, 2.0, rho, u);
+  if (active) {
 #pragma unroll
-    for (int i = 0; i < 27; ++i) fs[i] = (float)(f[i] - W27[i]);
-    ao = collide27_shifted(fs, a.beta, ac, 2.0, rho, u);
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < 27; ++i) static_cast<float*>(fout_)[(int64_t)i * n + k] = fs[i];
-    }
-    if (active && keep_alpha) alpha[k] = ao.alpha;
-    queue_far(a, kFarShards, active && ao.status == ALPHA_DEFER, (unsigned)k, ao.alpha);
-  } else {
-    ao = collide27_fp64(f, a.beta, ac, 2.0, rho, u);
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < 27; ++i) static_cast<double*>(fout_)[(int64_t)i * n + k] = f[i];
-    }
-    if (active && keep_alpha) alpha[k] = ao.alpha;
+    for (int i = 0; i < 27; ++i) pop(fout, i, nn, k) = f[i];
+    if (keep_alpha) alpha[k] = ao.alpha;
   }
+  if constexpr (kShifted)
+    queue_far(a, kFarShards, active && ao.status == ALPHA_DEFER, k, ao.alpha);
   wave_stats(stats, active, ao.iters, ao.status == ALPHA_DEFER ? -1 : ao.status, false,
              ao.logpath);
   if (active && nibb) {
