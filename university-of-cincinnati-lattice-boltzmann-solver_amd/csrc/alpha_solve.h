@@ -118,8 +118,8 @@ __device__ __forceinline__ double log1p_dev(double x) {
 // the absolute error is up to 1.2e-16: in g = sum f ((1+y) ln(1+y) - y) it
 // stays below the acceptance |g| <= tol S2 (tol 1e-10) while S2 > 1e-5 rho,
 // as on the far nodes this serves; a node below would report no convergence,
-// not a wrong root.  14 FP64 operations and two table reads where log1p_dev
-// takes about 30.
+// not a wrong root.  12 FP64 operations, a few on the high word and two
+// table reads where log1p_dev takes about 30.
 struct LogTable {
   double inv[64], L[64];
 };
@@ -131,9 +131,10 @@ __device__ __forceinline__ void log_table_entry(LogTable& t, int k) {
 }
 __device__ __forceinline__ double log1p_tab(double y, const LogTable& t) {
   const double u = 1.0 + y;
-  int e;
-  const double m = 2.0 * __builtin_frexp(u, &e);
-  const int k = (int)((m - 1.0) * 64.0);
+  // exponent, top six bits of the mantissa and m from the high word (u normal)
+  const int hi = __double2hiint(u);
+  const int k = (hi >> 14) & 63;
+  const double m = __hiloint2double((hi & 0x000fffff) | 0x3ff00000, __double2loint(u));
   const double r = fma(m, t.inv[k], -1.0);
   double p = 1.0 / 7.0;
   p = fma(p, r, -1.0 / 6.0);
@@ -144,8 +145,8 @@ __device__ __forceinline__ double log1p_tab(double y, const LogTable& t) {
   p = fma(p, r, 1.0);
   const double ln2_hi = 6.93147180369123816490e-01;
   const double ln2_lo = 1.90821492927058770002e-10;
-  const double de = (double)(e - 1);
-  return (de * ln2_hi + t.L[k]) + (de * ln2_lo + p * r);
+  const double de = (double)((hi >> 20) - 1023);
+  return fma(de, ln2_hi, t.L[k]) + fma(p, r, de * ln2_lo);
 }
 
 // The series as a polynomial: with C_n = (-1)^n S_n / (n (n-1)) and
@@ -222,80 +223,53 @@ __device__ __forceinline__ AlphaOut newton_alpha(Eval&& ev, double S2, double am
 // on direct logarithms evaluates g two to four times.  Bracket, bound and
 // iteration cap follow newton_alpha; iters counts the updates of the centre
 // or of the accepted root, as Newton counts its updates.
-// dx(i, d, x) yields D_i and x_i in FP64, fx(i) yields f_i; K = sum D ln(1+x).
-// kUnroll: unroll factor of the sweep over i (1 when dx / fx read memory).
-// lg(y): ln(1 + y) (log1p_dev or log1p_tab).
-template <int Q, int N, int kUnroll, class DX, class FX, class LG>
-__device__ __forceinline__ AlphaOut recentred_alpha(DX&& dx, FX&& fx, LG&& lg, double K, double S2,
-                                                    double amax, double alpha0, double tol,
-                                                    int maxit) {
+// sweep(a, w, first) fills a Sweep; the first one also gives K = sum D ln(1 + x)
+// (every lane's first sweep is the same one, so that the branch is uniform).
+template <int N>
+struct Sweep {
+  double K;
+  double g, gp;    // sum f ((1 + y) ln(1 + y) - y) and sum D ln(1 + y), y = a x
+  float zmax;      // max |z|
+  float T[N + 1];  // only steer the step (g and g' stay FP64 and decide
+                   // acceptance): FP32, their rounding in the bound below
+  bool edge;       // a at the positivity bound: some 1 + a x_i <= 0
+};
+template <int N, class SW>
+__device__ __forceinline__ AlphaOut recentred_alpha(SW&& sweep, double S2, double amax,
+                                                    double alpha0, double tol, int maxit) {
   double lo = 1.0, hi = amax < 1e6 ? amax : 1e6;
   bool hi_is_bound = amax < 1e6;
   double a = (alpha0 > lo && alpha0 < hi) ? alpha0 : 2.0;
   AlphaOut r{2.0, 0, ALPHA_NEWTON, true};
+  Sweep<N> w;
   for (int k = 0;; ++k) {
-    double g = 0.0, gp = 0.0, zmax = 0.0;
-    // the polynomial's coefficients only steer the step (g and g' stay FP64
-    // and decide acceptance), so they are summed in FP32; their rounding
-    // enters the acceptance bound below
-    float Tf[N + 1];
-#pragma unroll
-    for (int n = 2; n <= N; ++n) Tf[n] = 0.0f;
-    bool edge = false;  // a at the positivity bound: some 1 + a x_i <= 0
-#pragma unroll kUnroll
-    for (int i = 0; i < Q; ++i) {
-      double d, x;
-      dx(i, d, x);
-      const double f = fx(i);
-      const double y = a * x;
-      const double A = 1.0 + y;
-      if (A <= 0.0) { g -= f * y; edge = true; continue; }  // limit of (1+y) ln(1+y) at 0
-      const double la = lg(y);
-      g += f * (A * la - y);
-      gp += d * la;
-      const double z = x * drcp(A);
-      zmax = fmax(zmax, fabs(z));
-      const float zf = (float)z;
-      float t = (float)d * zf;
-      Tf[2] += t;
-#pragma unroll
-      for (int n = 3; n <= N; ++n) { t *= zf; Tf[n] += t; }
-    }
-    double T[N + 1];
-#pragma unroll
-    for (int n = 2; n <= N; ++n) T[n] = (double)Tf[n];
-    g -= a * K;
-    gp -= K;
+    sweep(a, w, k == 0);
+    const double g = fma(-a, w.K, w.g), gp = w.gp - w.K;
+    const double zmax = (double)w.zmax * (1.0 + 1e-6);  // not below the FP64 maximum
     if (fabs(g) <= tol * S2) { r.alpha = a; r.iters = k; return r; }
     if (g < 0.0 && a >= amax) { r.alpha = amax; r.iters = k; r.status = ALPHA_BOUND; return r; }
     if (k >= maxit) { r.alpha = a; r.iters = k; r.status = ALPHA_NOCONV; return r; }
     if (g < 0.0) lo = a; else { hi = a; hi_is_bound = false; }
-    if (edge) { a = 0.5 * (lo + hi); continue; }
-    // Newton on the polynomial from d = 0, |d| within the trust radius
-    const double rad = zmax > 0.0 ? 0.5 / zmax : 1e300;
+    if (w.edge) { a = 0.5 * (lo + hi); continue; }
+    // Newton on the polynomial p(d) = g + gp d + d^2 Q(d), Q = sum C_n d^(n-2),
+    // C_n = (-1)^n T_n / (n (n-1)), from d = 0, |d| within the trust radius
+    const double rad = zmax > 0.0 ? 0.5 * drcp(zmax) : 1e300;
     double dl = lo - a, dh = hi - a;
-    double dd = 0.0, p = g;
+    double dd = 0.0, p = g, pd = gp;
     bool ok = true;
     for (int j = 0; j < 8; ++j) {
-      double pd = gp, dn = dd;  // p'(d): gp + sum (-1)^n T_n d^(n-1) / (n-1)
-#pragma unroll
-      for (int n = 2; n <= N; ++n) {
-        const double tn = T[n] * dn / (n - 1.0);
-        pd += (n & 1) ? -tn : tn;
-        dn *= dd;
-      }
-      double st = dd - p / pd;
+      const double st = fma(-p, drcp(pd), dd);
       if (!(st > dl && st < dh) || fabs(st) > rad) { ok = false; dd = st; break; }
       dd = st;
-      // p(d) = g + gp d + sum (-1)^n T_n d^n / (n(n-1))
-      double pv = g + gp * dd, dn2 = dd * dd;
+      double q = (double)w.T[N] * (((N & 1) ? -1.0 : 1.0) / (N * (N - 1.0))), dq = 0.0;
 #pragma unroll
-      for (int n = 2; n <= N; ++n) {
-        const double tn = T[n] * dn2 / (n * (n - 1.0));
-        pv += (n & 1) ? -tn : tn;
-        dn2 *= dd;
+      for (int n = N - 1; n >= 2; --n) {
+        dq = fma(dq, dd, q);
+        q = fma(q, dd, (double)w.T[n] * (((n & 1) ? -1.0 : 1.0) / (n * (n - 1.0))));
       }
-      p = pv;
+      const double dQ = dd * q;
+      p = fma(dd, dQ + gp, g);
+      pd = fma(dd, fma(dd, dq, q + q), gp);
       if (fabs(p) <= 0.25 * tol * S2) break;
     }
     const double q = fabs(dd) * zmax;
@@ -304,16 +278,14 @@ __device__ __forceinline__ AlphaOut recentred_alpha(DX&& dx, FX&& fx, LG&& lg, d
       double qp = 1.0;
 #pragma unroll
       for (int n = 0; n < N - 1; ++n) qp *= q;
-      rem = T[2] * dd * dd * qp / (N * (N + 1.0) * (1.0 - q));
+      rem = (double)w.T[2] * dd * dd * qp * (1.0 / (N * (N + 1.0))) * drcp(1.0 - q);
       // the FP32 coefficients: relative error below 1e-6 (27 terms summed),
       // times the size of each polynomial term at dd
-      double dn = dd * dd, terms = 0.0;
+      double terms = 0.0;
 #pragma unroll
-      for (int n = 2; n <= N; ++n) {
-        terms += fabs(T[n]) * dn / (n * (n - 1.0));
-        dn *= fabs(dd);
-      }
-      rem += 1e-6 * terms;
+      for (int n = N; n >= 2; --n)
+        terms = fma(terms, fabs(dd), (double)fabsf(w.T[n]) * (1.0 / (n * (n - 1.0))));
+      rem = fma(1e-6 * dd * dd, terms, rem);
     }
     if (ok && fabs(p) + rem <= tol * S2) { r.alpha = a + dd; r.iters = k + 1; return r; }
     // next centre: the polynomial's step where it stays in the bracket and the

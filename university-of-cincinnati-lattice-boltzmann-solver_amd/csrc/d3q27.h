@@ -61,7 +61,7 @@ template <typename R>
 __device__ __forceinline__ R mul1(R a, R b) { return a + b + a * b; }
 
 // moments (FP64 sums), shifted equilibrium and D = feq~ - f~ with the mass
-// projection; shared by the streaming and far-from-equilibrium collides
+// projection; of the streaming collide and the learned features
 __device__ __forceinline__ void prep27_shifted(const float (&f)[27], float (&D)[27],
                                                double& rho_out, double (&u_out)[3]) {
   double r = 0.0, jx = 0.0, jy = 0.0, jz = 0.0;
@@ -218,11 +218,13 @@ __device__ __forceinline__ AlphaOut collide27_shifted(float (&f)[27], double bet
 // logarithmic solve of alpha_solve.h from the series seed, then relaxation.
 // Same moments, equilibrium and D as the streaming kernel formed for it.
 // f~ and D are parked in the block's LDS columns (stride kFarBlock = blockDim)
-// so the sweeps over the 27 directions run as loops unrolled by three (three
-// independent logarithms in flight) with few live registers; the relaxed
-// populations are written to fout~ at node.
+// so the sweeps over the 27 directions run as loops unrolled by three (three to
+// six independent logarithms in flight) with few live registers; the relaxed
+// populations are written to fout~ at node.  (Unrolled over all 27 with f and D
+// in registers, the compiler keeps what does not change between sweeps and
+// spills 340 registers.)
 constexpr int kRecentreOrder = 6;
-constexpr int kFarBlock = 64;
+constexpr int kFarBlock = 128;
 __device__ __forceinline__ AlphaOut collide27_far(float (&f)[27], double beta, const AlphaCfg& ac,
                                                   double seed, float* __restrict__ sf,
                                                   float* __restrict__ sD, bool active,
@@ -253,20 +255,35 @@ __device__ __forceinline__ AlphaOut collide27_far(float (&f)[27], double beta, c
   } else if (amax < 2.0) {
     ao = AlphaOut{amax, 0, ALPHA_BOUND, false};
   } else {
-    auto dx = [&](int i, double& d, double& x) __attribute__((always_inline)) {
-      d = (double)sD[i * kFarBlock];
-      x = d * drcp(W27[i] + (double)sf[i * kFarBlock]);
-    };
-    auto fx = [&](int i) __attribute__((always_inline)) { return W27[i] + (double)sf[i * kFarBlock]; };
-    auto lg = [&](double y) __attribute__((always_inline)) { return log1p_tab(y, lt); };
-    double K = 0.0;
+    ao = recentred_alpha<kRecentreOrder>(
+        [&](double a, Sweep<kRecentreOrder>& w, bool first) __attribute__((always_inline)) {
+          w.g = 0.0;
+          w.gp = 0.0;
+          w.zmax = 0.0f;
+          w.edge = false;
+          if (first) w.K = 0.0;
+#pragma unroll
+          for (int n = 2; n <= kRecentreOrder; ++n) w.T[n] = 0.0f;
 #pragma unroll 3
-    for (int i = 0; i < 27; ++i) {
-      double d, x;
-      dx(i, d, x);
-      K += d * lg(x);
-    }
-    ao = recentred_alpha<27, kRecentreOrder, 3>(dx, fx, lg, K, S2, amax, seed, ac.tol, ac.maxit);
+          for (int i = 0; i < 27; ++i) {
+            const float Di = sD[i * kFarBlock];
+            const double d = (double)Di, fi = W27[i] + (double)sf[i * kFarBlock];
+            const double x = d * drcp(fi);
+            if (first) w.K = fma(d, log1p_tab(x, lt), w.K);
+            const double y = a * x, A = 1.0 + y;
+            const bool edge = A <= 0.0;  // limit of (1 + y) ln(1 + y) at 0
+            w.edge |= edge;
+            const double la = edge ? 0.0 : log1p_tab(y, lt);
+            w.g = fma(fi, fma(A, la, -y), w.g);
+            w.gp = fma(d, la, w.gp);
+            const float z = edge ? 0.0f : (float)x * frcp((float)A);
+            w.zmax = fmaxf(w.zmax, fabsf(z));
+            float t = Di;
+#pragma unroll
+            for (int n = 2; n <= kRecentreOrder; ++n) { t *= z; w.T[n] += t; }
+          }
+        },
+        S2, amax, seed, ac.tol, ac.maxit);
   }
   const float ab = (float)(ao.alpha * beta);
   if (active) {

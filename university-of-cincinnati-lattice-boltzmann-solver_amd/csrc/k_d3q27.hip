@@ -278,59 +278,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 
 }
 
 // Far-from-equilibrium nodes queued by the streaming and boundary kernels
-// (max|x| beyond the in-register series): one thread per queued node reads
-// the pre-collision state stored in place, re-forms D, and solves for alpha by
-// the re-centred logarithmic sweeps from the series seed left in alpha[]; then
-// relaxes and stores.  The queue length stays on the device; the grid is
-// capped and strides over the queue, and blocks past its end leave at once.
-// Block 0 zeroes the other set of lengths, which the next step appends to.
-// One-wave blocks: the 13.8 KB of LDS per block lets three waves share a SIMD.
+// (max|x| beyond the in-register series): one lane per queued node reads the
+// pre-collision state stored in place, re-forms D, and solves for alpha by the
+// re-centred logarithmic sweeps from the queued series seed; then relaxes and
+// stores.  The queue length stays on the device; the blocks stride over the
+// queue, and those past its end leave once they have the lengths.  Block 0
+// zeroes the other set of lengths, which the next step appends to.
+constexpr int64_t kFarGrid = 2560;
 __global__ __launch_bounds__(kFarBlock) void k27_far(float* __restrict__ f_, double* __restrict__ alpha,
-                                               unsigned long long* __restrict__ stats, Box b,
-                                               StepArgs a, int keep_alpha) {
+                                                     unsigned long long* __restrict__ stats, Box b,
+                                                     StepArgs a, int keep_alpha) {
+  const int t = (int)threadIdx.x, l = t % 64, w = t / 64;
   // the next step's lengths start from zero (the previous far kernel read them)
   if (blockIdx.x == 0)
     for (unsigned s = threadIdx.x; s <= (unsigned)kFarShards; s += blockDim.x) a.defer_next[s] = 0u;
-  // the logarithm table, one entry per lane (kFarBlock = 64 entries)
+  // exclusive prefix of the shard lengths: thread t sums shards 2t and 2t + 1,
+  // the last one also shard kFarShards
+  __shared__ unsigned pre[kFarShards + 2], wsum[kFarBlock / 64];
   __shared__ LogTable lt;
-  log_table_entry(lt, (int)threadIdx.x);
-  // exclusive prefix of the shard lengths: lane l sums shards 5l .. 5l+4
-  __shared__ unsigned pre[kFarShards + 2];
+  __shared__ float sf[27 * kFarBlock], sD[27 * kFarBlock];
   {
-    constexpr int kPer = (kFarShards + 1 + 63) / 64;
-    static_assert(kFarBlock == 64 && kPer * 64 >= kFarShards + 1, "one wave scans the shards");
-    const int l = (int)threadIdx.x;
-    unsigned c[kPer], sum = 0;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int s = l * kPer + q;
-      c[q] = s <= kFarShards ? a.defer_count[s] : 0u;
-      sum += c[q];
-    }
-    unsigned inc = sum;
+    static_assert(kFarShards == 2 * kFarBlock, "two shards a thread");
+    const uint2 c = make_uint2(a.defer_count[2 * t], a.defer_count[2 * t + 1]);
+    const unsigned last = t == kFarBlock - 1 ? a.defer_count[kFarShards] : 0u;
+    unsigned inc = c.x + c.y;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const unsigned v = __shfl_up(inc, d);
       if (l >= d) inc += v;
     }
-    unsigned run = inc - sum;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int s = l * kPer + q;
-      if (s <= kFarShards + 1) pre[s] = run;
-      run += c[q];
+    if (l == 63) wsum[w] = inc;
+    __syncthreads();
+    for (int q = 0; q < w; ++q) inc += wsum[q];
+    pre[2 * t] = inc - c.x - c.y;
+    pre[2 * t + 1] = inc - c.y;
+    if (t == kFarBlock - 1) {
+      pre[kFarShards] = inc;
+      pre[kFarShards + 1] = inc + last;
     }
     __syncthreads();
   }
   const unsigned count = pre[kFarShards + 1];
-  const unsigned stride = gridDim.x * blockDim.x;
-  const unsigned first = blockIdx.x * blockDim.x;
+  if (blockIdx.x * (unsigned)kFarBlock >= count) return;
+  // the logarithm table, one entry per lane of the first wavefront
+  if (t < 64) log_table_entry(lt, t);
+  __syncthreads();
   const unsigned nn = (unsigned)b.n;
   AlphaCfg ac{a.tol, a.maxit, a.alpha_mode, a.thr};
-  __shared__ float sf[27 * kFarBlock], sD[27 * kFarBlock];
-  // grid-stride over the concatenated shards; whole blocks past the end leave at once
-  for (unsigned base = first; base < count; base += stride) {
-    const unsigned k = base + threadIdx.x;
+  for (unsigned base = blockIdx.x * (unsigned)kFarBlock; base < count;
+       base += gridDim.x * (unsigned)kFarBlock) {
+    const unsigned k = base + (unsigned)t;
     const bool active = k < count;
     const unsigned kk = active ? k : base;
     // shard holding entry kk: the last s with pre[s] <= kk
@@ -345,9 +342,8 @@ __global__ __launch_bounds__(kFarBlock) void k27_far(float* __restrict__ f_, dou
     float f[27];
 #pragma unroll
     for (int i = 0; i < 27; ++i) f[i] = (f_ + (size_t)i * nn)[node];
-    const double seed = (double)__uint_as_float(e.y);
-    AlphaOut ao = collide27_far(f, a.beta, ac, seed, sf + threadIdx.x, sD + threadIdx.x, active,
-                                f_, nn, node, lt);
+    const AlphaOut ao = collide27_far(f, a.beta, ac, (double)__uint_as_float(e.y), sf + t, sD + t,
+                                      active, f_, nn, node, lt);
     if (counted && keep_alpha) alpha[node] = ao.alpha;
     wave_stats(stats, counted, ao.iters, ao.status, false, ao.logpath);
   }
@@ -729,11 +725,7 @@ hipError_t launch_d3q27_init_uniform(const Box& b, void* f, int shifted, const u
 
 hipError_t launch_d3q27_far(const Box& b, void* fout, double* alpha, int keep_alpha,
                             unsigned long long* stats, const StepArgs& a, hipStream_t s) {
-  // up to 32768 one-wave blocks (enough for a 2M-node queue at one node per
-  // lane), grid-stride beyond; blocks past the queue's end leave at once.
-  // Measured on the C2 start-up: 2,560 blocks 350 us, 8,192 312 us, 32,768
-  // 304 us per launch.
-  const unsigned g = (unsigned)std::min<int64_t>(blocks_for(b.n, kFarBlock), 32768);
+  const unsigned g = (unsigned)std::min<int64_t>(blocks_for(b.n, kFarBlock), kFarGrid);
   k27_far<<<g, kFarBlock, 0, s>>>(static_cast<float*>(fout), alpha, stats, b, a, keep_alpha);
   return hipGetLastError();
 }
