@@ -246,8 +246,8 @@ __device__ __forceinline__ double alpha_estimate39(const S (*sf)[64], const doub
   return na;
 }
 
-// kMode 0: every node of the box (near-face nodes skipped when the box has
-// faces; with a link table, every node whose class is not 0); kMode 1: the
+// kMode 0: every node of a box with faces, walls or ghost nodes (near-face and
+// ghost nodes skipped; with a link table, every node whose class is not 0); kMode 1: the
 // listed near-face nodes, pulled through the face rules; kMode 2: the listed
 // wall nodes, their wall links taken from the rebuilt values of
 // k39_wall_rebuild and every other link pulled through the face rules.
@@ -1420,6 +1420,13 @@ hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s) {
     }
 #undef UCLBS_WALLS39
   }
+  // without faces, walls or ghost nodes the node updates of k_d3q39_open.hip
+  // (why the others keep this file's: there)
+  const bool open = !a.has_faces && !a.walls.cls && a.ghost == 0;
+  if (open) {
+    const hipError_t eo = launch_d3q39_step_open(b, a, s);
+    if (eo != hipSuccess) return eo;
+  }
 #define UCLBS_K39(F, SH, TU, KA, NR, NB)                                                         \
   hipLaunchKernelGGL((k39_step<F, SH, TU, KA, NR>), dim3(NB), dim3(64), 0, s, a.fin, a.gin,     \
                      a.fout, a.gout, a.lm, a.alpha, b, a.gas, a.ref, (long long)a.step, a.stats, \
@@ -1439,9 +1446,9 @@ hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s) {
   do {                      \
     if (a.gas.turbulent) UCLBS_K39_KA(F, SH, true); else UCLBS_K39_KA(F, SH, false); \
   } while (0)
-  if (a.fp32) {
+  if (!open && a.fp32) {
     if (a.shifted) UCLBS_K39_TU(true, true); else UCLBS_K39_TU(true, false);
-  } else {
+  } else if (!open) {
     if (a.shifted) UCLBS_K39_TU(false, true); else UCLBS_K39_TU(false, false);
   }
 #undef UCLBS_K39_TU

@@ -319,6 +319,8 @@ struct Step39 {
   Walls39 walls;        // cls == null: no link table
 };
 hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s);
+// the nodes of a level without faces, walls or ghost nodes (part of launch_d3q39_step)
+hipError_t launch_d3q39_step_open(const Box& b, const Step39& a, hipStream_t s);
 hipError_t launch_coarse_to_fine39(const void* cpf, const void* cnf, const void* cpg,
                                    const void* cng, const double* clm, const LevelMap& cm, void* ff,
                                    void* fg, double* flm, const LevelMap& fm,
