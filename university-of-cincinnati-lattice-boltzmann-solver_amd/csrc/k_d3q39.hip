@@ -1407,10 +1407,22 @@ hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s) {
   if (a.has_faces && a.n_near && !a.near_list) return hipErrorInvalidValue;
   const unsigned wall_blocks = (a.walls.n + 63u) / 64u;
   hipLaunchKernelGGL(k39_clear, dim3(1), dim3(1), 0, s, a.neg_count);
-  // the wall nodes' rebuilt populations, from the input buffers
-  if (a.walls.cls && a.walls.n) {
+  // the wall nodes on the side stream, beside the other nodes' launches: their
+  // rebuilt populations, from the input buffers, and their update.  A few
+  // hundred wavefronts, each a long chain: alone they left most of the chip
+  // idle (384 x 192 x 96 wedge: 306 + 241 us of a 5.9 ms step).  They write
+  // nodes and multipliers that no other launch touches.
+  const bool walls = a.walls.cls && a.walls.n;
+  hipStream_t ws = s;
+  if (walls && a.side) {
+    ws = a.side;
+    hipError_t ef = hipEventRecord(a.ev_fork, s);
+    if (ef == hipSuccess) ef = hipStreamWaitEvent(ws, a.ev_fork, 0);
+    if (ef != hipSuccess) return ef;
+  }
+  if (walls) {
 #define UCLBS_WALLS39(K)                                                                         \
-  hipLaunchKernelGGL(K, dim3(wall_blocks), dim3(64), 0, s, a.fin, a.gin, a.lm, b, a.gas, a.ref, \
+  hipLaunchKernelGGL(K, dim3(wall_blocks), dim3(64), 0, ws, a.fin, a.gin, a.lm, b, a.gas, a.ref, \
                      a.faces, (long long)a.step, a.walls, a.stats)
     if (a.shifted) {
       if (a.fp32) UCLBS_WALLS39(k39_wall_rebuild<true>); else UCLBS_WALLS39(k39_wall_rebuild<false>);
@@ -1427,16 +1439,16 @@ hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s) {
     const hipError_t eo = launch_d3q39_step_open(b, a, s);
     if (eo != hipSuccess) return eo;
   }
-#define UCLBS_K39(F, SH, TU, KA, NR, NB)                                                         \
-  hipLaunchKernelGGL((k39_step<F, SH, TU, KA, NR>), dim3(NB), dim3(64), 0, s, a.fin, a.gin,     \
+#define UCLBS_K39(F, SH, TU, KA, NR, NB, ST)                                                     \
+  hipLaunchKernelGGL((k39_step<F, SH, TU, KA, NR>), dim3(NB), dim3(64), 0, ST, a.fin, a.gin,    \
                      a.fout, a.gout, a.lm, a.alpha, b, a.gas, a.ref, (long long)a.step, a.stats, \
                      a.neg_count, a.neg_list, a.faces, a.has_faces, a.near_list, a.n_near,   \
                      a.ghost, a.walls)
 #define UCLBS_K39_FC(F, SH, TU, KA)                                              \
   do {                                                                           \
-    UCLBS_K39(F, SH, TU, KA, 0, blocks);                                         \
-    if (a.has_faces && a.n_near) UCLBS_K39(F, SH, TU, KA, 1, near_blocks);       \
-    if (a.walls.cls && a.walls.n) UCLBS_K39(F, SH, TU, KA, 2, wall_blocks);      \
+    if (walls) UCLBS_K39(F, SH, TU, KA, 2, wall_blocks, ws);                     \
+    UCLBS_K39(F, SH, TU, KA, 0, blocks, s);                                      \
+    if (a.has_faces && a.n_near) UCLBS_K39(F, SH, TU, KA, 1, near_blocks, s);    \
   } while (0)
 #define UCLBS_K39_KA(F, SH, TU) \
   do {                          \
@@ -1456,6 +1468,12 @@ hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s) {
 #undef UCLBS_K39_FC
 #undef UCLBS_K39
   hipError_t e = hipGetLastError();
+  if (ws != s) {
+    // also after an error, so that the side stream never runs on alone
+    hipError_t ej = hipEventRecord(a.ev_join, ws);
+    if (ej == hipSuccess) ej = hipStreamWaitEvent(s, a.ev_join, 0);
+    if (e == hipSuccess) e = ej;
+  }
   if (e != hipSuccess) return e;
   // repair pass over the nodes that produced a negative population; the
   // grids read the count on the device, so no host synchronisation is needed

@@ -317,6 +317,8 @@ struct Step39 {
   unsigned n_near;
   int ghost;            // depth of a refined level's ghost layer (not stepped), else 0
   Walls39 walls;        // cls == null: no link table
+  hipStream_t side;     // for the wall nodes, joined before the repair; null: none
+  hipEvent_t ev_fork, ev_join;
 };
 hipError_t launch_d3q39_step(const Box& b, const Step39& a, hipStream_t s);
 // the nodes of a level without faces, walls or ghost nodes (part of launch_d3q39_step)

@@ -602,6 +602,9 @@ int launch_steps39(Ctx* c, Level* L, int nsteps, hipEvent_t* ev) {
     a.walls.wf = L->wall_f;
     a.walls.wg = L->wall_g;
     a.walls.mach = c->gas39_mach;
+    a.side = c->side;
+    a.ev_fork = c->ev_fork;
+    a.ev_join = c->ev_join;
   }
   for (int s = 0; s < nsteps; ++s) {
     a.fin = L->f[L->cur];
