@@ -243,6 +243,7 @@ __global__ void k_collect_targets(const double* __restrict__ alpha, const unsign
 // Bound by the FP32 matrix rate and the chain of seven layer products with a
 // barrier after each: 206 MFMA a wavefront (2.8 us at 32 cycles each).
 constexpr int kTrainRows = 32;
+constexpr int kMaxRowBlocks = 256;
 constexpr int kTp = kTrainRows + 4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
@@ -250,12 +251,13 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// h = gelu(z), gp = gelu'(z) over one tanh
+// h = gelu(z), gp = gelu'(z): (1 + tanh u) / 2 = s = 1 / (1 + exp(-2 u)), so that
+// h = z s and gp = s + 2 z u' s (1 - s), over one exponential and one quotient
 __device__ __forceinline__ float gelu_both(float x, float& gp) {
   const float c = 0.7978845608028654f;
-  const float t = tanhf(c * (x + 0.044715f * x * x * x));
-  gp = 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * x * x);
-  return 0.5f * x * (1.0f + t);
+  const float s = 1.0f / (1.0f + expf(-2.0f * c * (x + 0.044715f * x * x * x)));
+  gp = fmaf(2.0f * c * x * s * (1.0f - s), 1.0f + 3.0f * 0.044715f * x * x, s);
+  return x * s;
 }
 
 // A operand of a forward product: W^T[o = 16 ot + l % 16][k], 16 k-steps
@@ -511,32 +513,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   }
 }
 
-// The gradient as the sum of nb blocks' parts, eight slices of the blocks a
+// The gradient as the sum of nb blocks' parts, 32 slices of the blocks a
 // weight (a fixed order, so the result is the same from run to run), and the
 // mean loss.  kAdam: applied to the parameters at once; else stored in g.
-// 32 weights a block: a slice's loads are 128 B rows of part.
+// 32 weights a block: a slice's loads are 128 B rows of part.  Bound by the
+// latency of a thread's loads, so that all of them (8 at 256 blocks) are in
+// flight; with 8 slices of up to 32 loads the launch took 11 us.
+constexpr int kSlices = 32;
 template <bool kAdam>
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ part,
-                                                    const double* __restrict__ lpart, int nb,
-                                                    int B, float* __restrict__ gout,
-                                                    double* __restrict__ loss,
-                                                    float* __restrict__ p, float* __restrict__ m,
-                                                    float* __restrict__ v, float lr, float c1,
-                                                    float c2) {
-  __shared__ float red[8][32];
+__global__ __launch_bounds__(32 * kSlices) void k_mlp_reduce(
+    const float* __restrict__ part, const double* __restrict__ lpart, int nb, int B,
+    float* __restrict__ gout, double* __restrict__ loss, float* __restrict__ p,
+    float* __restrict__ m, float* __restrict__ v, float lr, float c1, float c2) {
+  __shared__ float red[kSlices][33];
   __shared__ double lred[256];
   const int t = (int)threadIdx.x, c = t % 32, sl = t / 32;
   const int k = (int)blockIdx.x * 32 + c;
   float s = 0.0f;
   if (k < kMlpParams) {
-    const int per = (nb + 7) / 8, lo = sl * per, hi = min(nb, lo + per);
-    for (int b = lo; b < hi; ++b) s += part[(size_t)b * kMlpParams + k];
+    // blocks sl, sl + 32, ..: at most eight
+    static_assert(kMaxRowBlocks == 8 * kSlices && kMaxRowBlocks == 256, "slices, loss sums");
+    float q[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int b = sl + kSlices * j;
+      q[j] = b < nb ? part[(size_t)b * kMlpParams + k] : 0.0f;
+    }
+    s = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
   }
   red[sl][c] = s;
   if (blockIdx.x == 0) {
-    double a = 0.0;
-    for (int b = t; b < nb; b += 256) a += lpart[b];
-    lred[t] = a;
+    if (t < 256) lred[t] = t < nb ? lpart[t] : 0.0;
     __syncthreads();
     for (int d = 128; d > 0; d >>= 1) {
       if (t < d) lred[t] += lred[t + d];
@@ -545,17 +552,20 @@ __global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ pa
     if (t == 0) *loss = lred[0] / B;
   }
   __syncthreads();
-  if (t >= 32 || k >= kMlpParams) return;
-  const float gk = ((red[0][c] + red[1][c]) + (red[2][c] + red[3][c])) +
-                   ((red[4][c] + red[5][c]) + (red[6][c] + red[7][c]));
+  // a half-wavefront a weight adds its 32 slices
+  float gk = red[t % 32][t / 32];
+#pragma unroll
+  for (int d = 16; d > 0; d >>= 1) gk += __shfl_xor(gk, d);
+  const int kw = (int)blockIdx.x * 32 + t / 32;
+  if (t % 32 != 0 || kw >= kMlpParams) return;
   if constexpr (kAdam) {
-    const float mk = 0.9f * m[k] + 0.1f * gk;
-    const float vk = 0.999f * v[k] + 0.001f * gk * gk;
-    m[k] = mk;
-    v[k] = vk;
-    p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
+    const float mk = 0.9f * m[kw] + 0.1f * gk;
+    const float vk = 0.999f * v[kw] + 0.001f * gk * gk;
+    m[kw] = mk;
+    v[kw] = vk;
+    p[kw] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
   } else {
-    gout[k] = gk;
+    gout[kw] = gk;
   }
 }
 
@@ -848,7 +858,7 @@ hipError_t launch_mlp_targets(const double* alpha, MlpSamples& s, unsigned long 
 int mlp_blocks(int B) {
   // one block a CU (its weights and sums take 363 VGPRs, one wavefront a SIMD);
   // a block strides over the tiles beyond and keeps its weights and sums
-  return std::min((B + kTrainRows - 1) / kTrainRows, 256);
+  return std::min((B + kTrainRows - 1) / kTrainRows, kMaxRowBlocks);
 }
 
 // forward + backward of one batch (X: B x 12, y: B targets); gradients into g
@@ -858,7 +868,7 @@ hipError_t launch_mlp_loss_grad(const float* P, const float* X, const float* y, 
   const int nb = mlp_blocks(B);
   hipLaunchKernelGGL(k_mlp_rows<kRowsGrad>, dim3(nb), dim3(256), 0, st, P, X, y, B, 0ull,
                      (uint64_t)0, (uint64_t)0, w.part, w.loss, (float*)nullptr);
-  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 31) / 32), dim3(256), 0, st, w.part,
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 31) / 32), dim3(32 * kSlices), 0, st, w.part,
                      w.loss, nb, B, g, loss, (float*)nullptr, (float*)nullptr, (float*)nullptr,
                      0.0f, 0.0f, 0.0f);
   return hipGetLastError();
@@ -873,7 +883,7 @@ hipError_t launch_mlp_train_step(float* P, float* m, float* v, const float* X, c
   const float c1 = 1.0f - powf(0.9f, (float)t), c2 = 1.0f - powf(0.999f, (float)t);
   hipLaunchKernelGGL(k_mlp_rows<kRowsGather>, dim3(nb), dim3(256), 0, st, P, X, y, B, n, seed, step,
                      w.part, w.loss, (float*)nullptr);
-  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 31) / 32), dim3(256), 0, st, w.part,
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 31) / 32), dim3(32 * kSlices), 0, st, w.part,
                      w.loss, nb, B, (float*)nullptr, loss, P, m, v, lr, c1, c2);
   return hipGetLastError();
 }
