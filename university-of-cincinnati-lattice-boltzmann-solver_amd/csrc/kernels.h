@@ -88,6 +88,11 @@ struct BvhNode {
   int32_t a, b;
 };
 
+// a triangle's plane and edge lines (k_links.hip, cast_wave)
+struct TriPlane {
+  double n[3], dot, line[3][3], moment[3][3];
+};
+
 struct LinkGeom {
   Box box;
   double origin[3];
@@ -105,6 +110,8 @@ struct LinkGeom {
   // the box centre
   double ray[3];
   double ray_len;
+  const TriPlane* plane;  // [ntri]
+  double reach;           // no |coordinate sum| of node or triangle is larger
 };
 
 // Builds the hierarchy on the host (median split of the longest centroid axis,
@@ -115,6 +122,8 @@ int build_bvh(const double* tbb, int ntri, std::vector<BvhNode>* nodes,
               std::vector<int32_t>* idx);
 constexpr int kBvhMaxDepth = 38;
 
+hipError_t launch_tri_planes(const double* tri, const double* nrm, int ntri, TriPlane* out,
+                             hipStream_t s);
 hipError_t launch_build_links27(const LinkGeom& g, int32_t* state, unsigned long long* counts,
                                 hipStream_t s);
 hipError_t launch_build_links39(const LinkGeom& g, int32_t* state, unsigned long long* counts,

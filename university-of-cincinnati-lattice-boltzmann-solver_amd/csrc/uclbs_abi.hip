@@ -1595,6 +1595,8 @@ int uclbs_build_links(void* ctx, int lvl, const double origin[3], double dx, int
   if (e == hipSuccess) e = hipMalloc(&dnrm, nt * 3 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&dtbb, nt * 6 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&dcnt, 2 * sizeof(unsigned long long));
+  uclbs::TriPlane* dplane = nullptr;
+  if (e == hipSuccess) e = hipMalloc(&dplane, nt * sizeof(uclbs::TriPlane));
   if (e == hipSuccess && ntri) e = hipMemcpy(dtri, tri, (size_t)ntri * 9 * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess && ntri) e = hipMemcpy(dnrm, nrm, (size_t)ntri * 3 * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dtbb, tbb.data(), nt * 6 * sizeof(double), hipMemcpyHostToDevice);
@@ -1607,7 +1609,19 @@ int uclbs_build_links(void* ctx, int lvl, const double origin[3], double dx, int
     g.tbb = dtbb;
     g.bvh = dbvh;
     g.bvh_idx = dbidx;
-    if (L->multibox) {
+    g.plane = dplane;
+    e = uclbs::launch_tri_planes(dtri, dnrm, g.ntri, dplane, c->stream);
+    for (int d = 0; d < 3; ++d) {
+      const int ext[3] = {g.box.nx, g.box.ny, g.box.nz};
+      double far = std::max(std::fabs(origin[d]), std::fabs(origin[d] + (double)(ext[d] - 1) * dx));
+      if (ntri) far = std::max(far, std::max(std::fabs(gbb[2 * d]), std::fabs(gbb[2 * d + 1])));
+      for (size_t b = 0; L->multibox && b < L->hbox.size(); ++b)
+        far = std::max(far, std::max(std::fabs(origin[d] + (double)(L->blo[3 * b + d] - 1) * dx),
+                                     std::fabs(origin[d] + (double)(L->bhi[3 * b + d] + 1) * dx)));
+      g.reach += far;
+    }
+    if (e != hipSuccess) {
+    } else if (L->multibox) {
       // box by box: the box's stored nodes (ghost shell included) at level
       // position blo - 1 + (a, b, c), i.e. origin + (blo - 1 + (a, b, c)) dx;
       // built into a scratch table and placed at the box's offset
@@ -1676,6 +1690,7 @@ int uclbs_build_links(void* ctx, int lvl, const double origin[3], double dx, int
   (void)hipFree(dtbb);
   (void)hipFree(dbvh);
   (void)hipFree(dbidx);
+  (void)hipFree(dplane);
   (void)hipFree(dcnt);
   if (e != hipSuccess) return set_err(UCLBS_E_HIP, "build_links failed: %s", hipGetErrorString(e));
   if (q39) {
