@@ -9,6 +9,7 @@
 #include <cstring>
 #include <string>
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -166,6 +167,8 @@ struct Ctx {
   hipStream_t stream = nullptr;
   hipStream_t side = nullptr;  // boundary-list kernel, concurrent with the streaming kernel
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_fork = nullptr, ev_join = nullptr;
+  void* pin[4] = {};         // pinned pieces of to_host and their events
+  hipEvent_t pin_ev[4] = {};
   std::vector<Level> levels;
   unsigned long long* d_stats = nullptr;
   // inlet / outlet / freestream equilibria (full FP64 populations)
@@ -561,6 +564,63 @@ int resolve_bc39(Ctx* c, Level* L, uclbs::Faces39* fc) {
   return UCLBS_OK;
 }
 
+// Copy of a finished device array to pageable host memory.  A single pageable
+// copy is bound by one thread that moves 8 GB/s from its staging buffer into
+// pages it touches first; here four threads take pieces in turn, each through a
+// pinned buffer of its own (kept with the context, 16 MB).  106 MB: 13 -> 5 ms.
+// Small copies, and any failure to get buffers or threads, take the single copy.
+constexpr int kCopyThreads = 4;
+constexpr size_t kCopyPiece = (size_t)4 << 20;
+
+bool copy_buffers(Ctx* c) {
+  for (int t = 0; t < kCopyThreads; ++t) {
+    if (!c->pin[t] && hipHostMalloc(&c->pin[t], kCopyPiece, hipHostMallocDefault) != hipSuccess) {
+      c->pin[t] = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    if (!c->pin_ev[t] &&
+        hipEventCreateWithFlags(&c->pin_ev[t], hipEventDisableTiming) != hipSuccess) {
+      c->pin_ev[t] = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  return true;
+}
+
+hipError_t to_host(Ctx* c, void* dst, const void* src, size_t bytes) {
+  if (bytes < 4 * kCopyPiece || !copy_buffers(c))
+    return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+  std::atomic<size_t> next{0};
+  std::atomic<int> failed{(int)hipSuccess};
+  auto work = [&](int t) {
+    hipError_t e = hipSetDevice(c->device);
+    for (;;) {
+      const size_t at = next.fetch_add(kCopyPiece);
+      if (at >= bytes) break;  // also after a failure elsewhere: pieces are few
+      const size_t m = std::min(kCopyPiece, bytes - at);
+      if (e == hipSuccess)
+        e = hipMemcpyAsync(c->pin[t], static_cast<const char*>(src) + at, m, hipMemcpyDeviceToHost,
+                           c->stream);
+      if (e == hipSuccess) e = hipEventRecord(c->pin_ev[t], c->stream);
+      if (e == hipSuccess) e = hipEventSynchronize(c->pin_ev[t]);
+      if (e != hipSuccess) break;
+      std::memcpy(static_cast<char*>(dst) + at, c->pin[t], m);
+    }
+    if (e != hipSuccess) failed = (int)e;
+  };
+  std::thread helper[kCopyThreads];
+  int made = 1;
+  try {
+    for (; made < kCopyThreads; ++made) helper[made] = std::thread(work, made);
+  } catch (...) {  // no more threads: the ones there are take all pieces
+  }
+  work(0);
+  for (int t = 1; t < made; ++t) helper[t].join();
+  return (hipError_t)failed.load();
+}
+
 int launch_steps39(Ctx* c, Level* L, int nsteps, hipEvent_t* ev) {
   uclbs::Step39 a{};
   a.gas = L->gas39;
@@ -802,6 +862,10 @@ int uclbs_destroy(void* ctx) {
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->side) { (void)hipStreamSynchronize(c->side); (void)hipStreamDestroy(c->side); }
+  for (void* p : c->pin)
+    if (p) (void)hipHostFree(p);
+  for (hipEvent_t e : c->pin_ev)
+    if (e) (void)hipEventDestroy(e);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1736,8 +1800,7 @@ int uclbs_download_links(void* ctx, int lvl, int32_t* state, int64_t n_nodes) {
   if (!L->state) return set_err(UCLBS_E_STATE, "level %d has no link table", lvl);
   if (!state || n_nodes != L->box.n) return set_err(UCLBS_E_ARG, "download_links: wrong node count");
   if ((rc = set_device(c))) return rc;
-  HIP_TRY(hipMemcpy(state, L->state, (size_t)n_nodes * q_of(c) * sizeof(int32_t),
-                    hipMemcpyDeviceToHost));
+  HIP_TRY(to_host(c, state, L->state, (size_t)n_nodes * q_of(c) * sizeof(int32_t)));
   return UCLBS_OK;
 }
 
