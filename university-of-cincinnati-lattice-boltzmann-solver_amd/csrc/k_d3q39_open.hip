@@ -10,8 +10,9 @@
 // collision where it took 4,500.
 //
 // 65 x 48 x 33, FP32 storage: 116 -> 83 us a step; 96 x 80 x 64 shifted, FP64
-// storage: 861 -> 399 us (there g is not staged in LDS, so that four blocks fit
-// a CU instead of two).  Distance from 64-bit results: 1.6e-9 as before, 1.4e-14
+// storage: 861 -> 340 us (there g is not staged in LDS, so that four blocks fit
+// a CU instead of two, and is read again ahead of alpha: 399 us where the
+// collision waited for it).  Distance from 64-bit results: 1.6e-9 as before, 1.4e-14
 // -> 1.2e-14.
 //
 // Levels with faces, walls or ghost nodes keep k_d3q39.hip's summation order:
@@ -254,17 +255,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
              (unsigned)nx * ((unsigned)wrapm(y - CY39[i], ny) +
                              (unsigned)ny * (unsigned)wrapm(z - CZ39[i], nz));
     };
+    // at one wavefront a SIMD every wait shows: the multipliers are asked for
+    // with the populations
+    double lm[kM39];
+#pragma unroll
+    for (int k = 0; k < kM39; ++k) lm[k] = lmv[(size_t)k * n + node];
 #pragma unroll
     for (int i = 0; i < Q39; ++i) {
       const unsigned src = source(i);
       sf[i][t] = fA[(size_t)i * n + src];
       if constexpr (kStageG) sg[i][t] = gA[(size_t)i * n + src];
     }
-    // g of direction i, from LDS or where it was pulled from
+    // g of direction i, from LDS or from registers (read where it is pulled from,
+    // for the moments, and again for the collision)
+    S gr[kStageG ? 1 : Q39];
     auto g_of = [&](int i) __attribute__((always_inline)) {
       if constexpr (kStageG) return (double)sg[i][t];
-      else return (double)gA[(size_t)i * n + source(i)];
+      else return (double)gr[i];
     };
+    auto read_g = [&]() __attribute__((always_inline)) {
+      if constexpr (!kStageG) {
+#pragma unroll
+        for (int i = 0; i < Q39; ++i) gr[i] = gA[(size_t)i * n + source(i)];
+      }
+    };
+    read_g();
     double rho = 0.0, mx = 0.0, my = 0.0, mz = 0.0, en = 0.0;
 #pragma unroll
     for (int i = 0; i < Q39; ++i) {
@@ -286,9 +301,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
                              rho * (T + u[1] * u[1]), rho * (T + u[2] * u[2]), rho * u[0] * u[1],
                              rho * u[0] * u[2], rho * u[1] * u[2], qf * u[0], qf * u[1],
                              qf * u[2]};
-    double lm[kM39], dp[kM39];
-#pragma unroll
-    for (int k = 0; k < kM39; ++k) lm[k] = lmv[(size_t)k * n + node];
+    double dp[kM39];
     // the last iteration's equilibrium stays in LDS for alpha and collision
     const ExpTab39 ex{etab};
     const int it = lm_newton39_groups<kShifted>(
@@ -299,6 +312,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 #pragma unroll
     for (int k = 0; k < kM39; ++k) lmv[(size_t)k * n + node] = lm[k];
 
+    // asked for before alpha, which hides the wait; Newton has no registers for it
+    __asm__ volatile("" ::: "memory");
+    read_g();
     double dim_mu, dim_temp;
     const double mu = sutherland_open39(T, gs, &dim_mu, &dim_temp);
     double al = 2.0;
