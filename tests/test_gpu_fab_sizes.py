@@ -1,6 +1,6 @@
 """Device FArrayBox exchange at the sizes where its two kernels can go wrong:
-boxes of one node, of one block and one node more, odd extents, ghost widths 0
-to 3, both lattices and storage forms.  Import then export returns the values
+the smallest boxes that a level takes (five nodes an axis on D3Q39), rows around
+the block size, whole blocks, odd extents, ghost widths 0 to 3, both lattices and storage forms.  Import then export returns the values
 in storage precision (exactly in FP64; one FP32 rounding of the deviation in
 FP32), leaves ghost cells alone, and fills both population buffers (a step
 reads one and a download of the next reads the other)."""
@@ -14,8 +14,8 @@ from test_gpu_fab import Fab, _hip
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape,ghost", [((1, 1, 1), 0), ((1, 1, 1), 3), ((255, 1, 1), 1),
-                                         ((257, 1, 1), 0), ((5, 3, 17), 2), ((64, 4, 1), 0),
+@pytest.mark.parametrize("shape,ghost", [((5, 5, 5), 0), ((5, 5, 5), 3), ((255, 5, 5), 1),
+                                         ((257, 5, 5), 0), ((5, 7, 17), 2), ((64, 8, 5), 0),
                                          ((33, 9, 7), 1)])
 @pytest.mark.parametrize("lattice", ["d3q27", "d3q39"])
 @pytest.mark.parametrize("precision", ["fp32s", "fp64"])
