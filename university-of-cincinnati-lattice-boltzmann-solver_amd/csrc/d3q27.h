@@ -61,7 +61,8 @@ template <typename R>
 __device__ __forceinline__ R mul1(R a, R b) { return a + b + a * b; }
 
 // moments (FP64 sums), shifted equilibrium and D = feq~ - f~ with the mass
-// projection; of the streaming collide and the learned features
+// projection; shared by the streaming and far-from-equilibrium collides and
+// the learned features
 __device__ __forceinline__ void prep27_shifted(const float (&f)[27], float (&D)[27],
                                                double& rho_out, double (&u_out)[3]) {
   double r = 0.0, jx = 0.0, jy = 0.0, jz = 0.0;

@@ -241,7 +241,9 @@ __global__ void k_collect_targets(const double* __restrict__ alpha, const unsign
 // column, the weight gradients, which contract over the rows, by float4.  Each
 // wavefront reads its half of a weight matrix once, into registers.
 // Bound by the FP32 matrix rate and the chain of seven layer products with a
-// barrier after each: 206 MFMA a wavefront (2.8 us at 32 cycles each).
+// barrier after each: 206 MFMA a wavefront (2.8 us at 32 cycles each) of the
+// 17 us that the launch takes at 8,192 rows; the rest is the draw of the rows,
+// two dependent reads and the barriers.  Before: 490 us a step in 18 launches.
 constexpr int kTrainRows = 32;
 constexpr int kMaxRowBlocks = 256;
 constexpr int kTp = kTrainRows + 4;
@@ -570,7 +572,8 @@ __global__ __launch_bounds__(32 * kSlices) void k_mlp_reduce(
 }
 
 // mean and standard deviation of the targets in FP64: a block's sums, then
-// one block over the blocks (one block over all of 786k targets ran for 1.6 ms)
+// one block over the blocks (with one block over all of 786k targets the first
+// training on them took 2 ms longer than the next)
 constexpr int kMomentBlocks = 256;
 __device__ __forceinline__ void sum2_256(double& a, double& b) {
   __shared__ double s1[256], s2[256];
