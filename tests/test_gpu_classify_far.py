@@ -1,8 +1,11 @@
 """The wavefront-wide solid test where its shortcut must not answer: triangles
 whose planes hold nodes or rays, rays through vertices and along edges (a body
 aligned with the grid and centred on it), a body far from the origin, small and
-ragged boxes, a body much larger and much smaller than the box.  The table, the
-solid count and the tie count equal the CPU restatement's exactly."""
+ragged boxes, a body much larger and much smaller than the box; geometries in
+small units (spacing 1e-3 to 1e-6) and normals that are not unit vectors, where
+the absolute tolerances of the crossing test (1.24e-16 on volumes, 1e-14 on a
+plane through the node) decide many candidates.  The table, the solid count and
+the tie count equal the CPU restatement's exactly."""
 import numpy as np
 import pytest
 
@@ -60,7 +63,29 @@ CASES = {
 @pytest.mark.parametrize("name", list(CASES))
 def test_table_equals_cpu(pkg, orc, name):
     shape, origin, dx, tri, centre = CASES[name]
+    compare(pkg, orc, name, shape, origin, dx, tri, normals(tri, np.array(centre)))
+
+
+@pytest.mark.parametrize("dx", [1e-3, 1e-4, 3e-5, 1e-5, 1e-6])
+@pytest.mark.parametrize("name", ["sphere off the nodes", "box on half nodes", "sphere of many triangles"])
+def test_small_units_equal_cpu(pkg, orc, name, dx):
+    if name in CASES:
+        shape, _, _, tri, centre = CASES[name]
+    else:
+        shape, centre = (48, 40, 32), (23.31, 19.47, 15.82)
+        tri = octahedron(np.array(centre), 9.0, 5)
     nrm = normals(tri, np.array(centre))
+    compare(pkg, orc, f"{name}, dx {dx}", shape, (0, 0, 0), dx, tri * dx, nrm)
+
+
+@pytest.mark.parametrize("length", [1e-12, 1e-8, 1e6])
+def test_normals_of_any_length_equal_cpu(pkg, orc, length):
+    shape, origin, dx, tri, centre = CASES["sphere off the nodes"]
+    compare(pkg, orc, f"normals of length {length}", shape, origin, dx, tri,
+            length * normals(tri, np.array(centre)))
+
+
+def compare(pkg, orc, name, shape, origin, dx, tri, nrm):
     s = pkg.Solver(precision="fp32s", nu=0.01)
     s.define_level(0, shape, periodic=(0, 0, 0))
     s.set_faces(0, FACES)

@@ -17,9 +17,9 @@
 //     neighbour's node code (:687-716); a solid node gets -666 everywhere (:87).
 // Ties that make the reference re-cast with a time-seeded random ray
 // (utilities/ray_casting.f95) are re-cast here along three fixed directions
-// and counted.  One thread per node; the triangle soup and its bounding boxes
-// are read in index order by every thread (the same addresses across a
-// wavefront, so they stream through the cache).  The arithmetic is written in
+// and counted.  One thread per node; triangles are found through a hierarchy of
+// their bounding boxes, which the node codes walk once for a wavefront
+// (cast_wave) and the links once a thread.  The arithmetic is written in
 // the reference's expression order with contraction off, so the table is
 // bit-identical to the CPU restatement.
 #pragma clang fp contract(off)
@@ -214,9 +214,14 @@ __global__ __launch_bounds__(256) void k_tri_planes(const double* __restrict__ t
 // volumes are pc |e2 - e1| times those products.  With coordinates up to
 // g.reach = R, rounding moves a product by less than 1e-14 R^2 and a volume by
 // less than 1e-15 R^3; the test asks for products beyond 1e-12 R^2 and a plane
-// at least R / 100 along the ray, hence volumes beyond 1e-14 R^3.  Anything
-// nearer, a ray nearly in the plane or a plane through its end (where a tie may
-// be) takes cast_parity's expressions.
+// at least R / 100 along the ray, hence volumes beyond 1e-14 R^3.  cast_parity's
+// own tolerances are absolute (kPlusEps on volumes and on lower, kVSmall on
+// upper), whatever the unit of length: so the products are also beyond
+// 4e-16 / (R / 100), which puts the volumes beyond 3 kPlusEps, and upper and
+// lower, the same numbers there, beyond their limits.  Anything nearer, a ray
+// nearly in the plane or a plane through its end (where a tie may be) takes
+// cast_parity's expressions; so does every candidate of a geometry whose products
+// stay below that (R of 1e-4 and less).
 // Bound by FP64 issue, ~40 operations a candidate and wavefront.  128 x 96 x 80
 // nodes and 20,480 triangles: 22.3 -> 6.0 ms, against one walk a node with every
 // candidate's crossing point and volumes formed.
@@ -235,7 +240,8 @@ __device__ int cast_wave(const LinkGeom& g, const double* e1, const double* e2, 
   F[0] = e1[1] * d[2] - e1[2] * d[1];
   F[1] = e1[2] * d[0] - e1[0] * d[2];
   F[2] = e1[0] * d[1] - e1[1] * d[0];
-  const double clear = 1e-12 * g.reach * g.reach, near = 1e-2 * g.reach;
+  const double near = 1e-2 * g.reach;
+  const double clear = fmax(1e-12 * g.reach * g.reach, 4e-16 / near);
   // box_out over the segment's extremes
   auto inside = [&](const double* bb) __attribute__((always_inline)) {
     bool in = true;
@@ -275,7 +281,8 @@ __device__ int cast_wave(const LinkGeom& g, const double* e1, const double* e2, 
       const bool down = w[0] < -clear || w[1] > clear || w[2] < -clear;
       const bool sure = fabs(w[0]) > clear && fabs(w[1]) > clear && fabs(w[2]) > clear;
       const bool miss = up && down && sure && fabs(upper) * len >= near * fabs(lower) &&
-                        fabs(lower) > 1.0e-9 * len && fabs(upper - lower) > 1.0e-12;
+                        fabs(lower) > 1.0e-9 * len && fabs(upper - lower) > 1.0e-12 &&
+                        fabs(lower) > 4.0 * kPlusEps && fabs(upper) > 4.0 * kVSmall;
       if (!__any(in && !miss)) continue;
       if (in && !miss) {
         if (lower >= kMinusEps && lower <= kPlusEps) {
