@@ -17,6 +17,7 @@
 #include "../../include/uclbs_hip.h"
 #include "kernels.h"
 #include "lattice.h"
+#include "link_reach.h"
 #include "philox.h"
 #include "cluster.h"
 
@@ -1676,15 +1677,9 @@ int uclbs_build_links(void* ctx, int lvl, const double origin[3], double dx, int
     g.bvh_idx = dbidx;
     g.plane = dplane;
     e = uclbs::launch_tri_planes(dtri, dnrm, g.ntri, dplane, c->stream);
-    for (int d = 0; d < 3; ++d) {
-      const int ext[3] = {g.box.nx, g.box.ny, g.box.nz};
-      double far = std::max(std::fabs(origin[d]), std::fabs(origin[d] + (double)(ext[d] - 1) * dx));
-      if (ntri) far = std::max(far, std::max(std::fabs(gbb[2 * d]), std::fabs(gbb[2 * d + 1])));
-      for (size_t b = 0; L->multibox && b < L->hbox.size(); ++b)
-        far = std::max(far, std::max(std::fabs(origin[d] + (double)(L->blo[3 * b + d] - 1) * dx),
-                                     std::fabs(origin[d] + (double)(L->bhi[3 * b + d] + 1) * dx)));
-      g.reach += far;
-    }
+    const int extent[3] = {g.box.nx, g.box.ny, g.box.nz};
+    g.reach = uclbs::link_reach(origin, dx, extent, L->multibox ? L->hbox.size() : 0,
+                                L->blo.data(), L->bhi.data(), ntri ? gbb : nullptr);
     if (e != hipSuccess) {
     } else if (L->multibox) {
       // box by box: the box's stored nodes (ghost shell included) at level
