@@ -274,6 +274,16 @@ __host__ __device__ inline double kfit39(double ak, double bk, double ck, double
   return exp(ak * k4 + bk * k3 + ck * k2 + dk * kek + ek);
 }
 
+// The fits' coefficients up to 2250 K and up to 4250 K, each for three bands of
+// pressure (0.1-10, 10-100, 100-1000), as argument lists: as arrays they move
+// the inliner, and k39_step_open takes 1% longer
+#define UCLBS_KAPPA_UP_TO_2250K_0 0.334316, 3.28202, 11.9939, 20.0944, 4.62882
+#define UCLBS_KAPPA_UP_TO_2250K_1 0.413573, 3.83393, 13.1885, 20.7305, 4.27728
+#define UCLBS_KAPPA_UP_TO_2250K_2 0.208749, 1.92122, 6.58813, 10.7630, -1.27699
+#define UCLBS_KAPPA_UP_TO_4250K_0 10.9992, 387.106, 387.282, 5.48304, -1.20106
+#define UCLBS_KAPPA_UP_TO_4250K_1 82.1184, 308.927, 423.174, 250.668, 47.5889
+#define UCLBS_KAPPA_UP_TO_4250K_2 38.8677, 123.284, 144.224, 72.8083, 0.684807
+
 // quick_calcs.f95:70-215 with kappa_bottom = kappa_ref; false where the
 // reference calls error_out
 __host__ __device__ inline bool therm_cond39(double rho, double T, const Gas39& g, double* kappa) {
@@ -287,18 +297,59 @@ __host__ __device__ inline bool therm_cond39(double rho, double T, const Gas39& 
   }
   if (unit_temp <= 2250.0) {
     unit_p = unit_rho * g.R * unit_temp / 101300.0;
-    if (unit_p < 10.0 && unit_p > 0.1) { *kappa = kfit39(0.334316, 3.28202, 11.9939, 20.0944, 4.62882, unit_temp) / kb; return true; }
-    if (unit_p > 10.0 && unit_p < 100.0) { *kappa = kfit39(0.413573, 3.83393, 13.1885, 20.7305, 4.27728, unit_temp) / kb; return true; }
-    if (unit_p > 100.0 && unit_p < 1000.0) { *kappa = kfit39(0.208749, 1.92122, 6.58813, 10.7630, -1.27699, unit_temp) / kb; return true; }
+    if (unit_p < 10.0 && unit_p > 0.1) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_2250K_0, unit_temp) / kb; return true; }
+    if (unit_p > 10.0 && unit_p < 100.0) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_2250K_1, unit_temp) / kb; return true; }
+    if (unit_p > 100.0 && unit_p < 1000.0) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_2250K_2, unit_temp) / kb; return true; }
     return false;
   }
   if (unit_temp <= 4250.0) {
-    if (unit_p < 10.0 && unit_p > 0.1) { *kappa = kfit39(10.9992, 387.106, 387.282, 5.48304, -1.20106, unit_temp) / kb; return true; }
-    if (unit_p > 10.0 && unit_p < 100.0) { *kappa = kfit39(82.1184, 308.927, 423.174, 250.668, 47.5889, unit_temp) / kb; return true; }
-    if (unit_p > 100.0 && unit_p < 1000.0) { *kappa = kfit39(38.8677, 123.284, 144.224, 72.8083, 0.684807, unit_temp) / kb; return true; }
+    if (unit_p < 10.0 && unit_p > 0.1) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_4250K_0, unit_temp) / kb; return true; }
+    if (unit_p > 10.0 && unit_p < 100.0) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_4250K_1, unit_temp) / kb; return true; }
+    if (unit_p > 100.0 && unit_p < 1000.0) { *kappa = kfit39(UCLBS_KAPPA_UP_TO_4250K_2, unit_temp) / kb; return true; }
     return false;
   }
   return false;
 }
+
+// therm_cond39 without a branch of its own for any lane: uniform branches and
+// selects, so that the wavefront stays whole (why k39_step needs that: there)
+__device__ inline bool therm_cond_wave39(double rho, double T, const Gas39& g, double* kappa) {
+  const double kb = g.kappa_ref;
+  const double unit_temp = T * g.t_ref * g.gama;
+  const double unit_rho = rho * g.rho_ref;
+  const bool low = unit_temp <= 500.0, mid = unit_temp <= 2250.0;
+  const double unit_p = mid ? unit_rho * g.R * unit_temp / 101300.0 : unit_temp * unit_rho * g.R;
+  const bool p0 = unit_p < 10.0 && unit_p > 0.1, p1 = unit_p > 10.0 && unit_p < 100.0,
+             p2 = unit_p > 100.0 && unit_p < 1000.0;
+  const bool fit = !low && unit_temp <= 4250.0 && (p0 || p1 || p2);
+  double k = 0.0;
+  if (__any(low)) {
+    const double v =
+        418.1 * (5.9776e-6 * pow(unit_temp, 1.5) / (unit_temp + (double)194.4f)) / kb;
+    k = low ? v : k;
+  }
+  if (__any(fit)) {
+    const double fits[6][5] = {{UCLBS_KAPPA_UP_TO_2250K_0}, {UCLBS_KAPPA_UP_TO_2250K_1},
+                               {UCLBS_KAPPA_UP_TO_2250K_2}, {UCLBS_KAPPA_UP_TO_4250K_0},
+                               {UCLBS_KAPPA_UP_TO_4250K_1}, {UCLBS_KAPPA_UP_TO_4250K_2}};
+    double c[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      const double m = p0 ? fits[0][j] : p1 ? fits[1][j] : fits[2][j];
+      const double h = p0 ? fits[3][j] : p1 ? fits[4][j] : fits[5][j];
+      c[j] = mid ? m : h;
+    }
+    const double v = kfit39(c[0], c[1], c[2], c[3], c[4], unit_temp) / kb;
+    k = fit ? v : k;
+  }
+  *kappa = k;
+  return low || fit;
+}
+#undef UCLBS_KAPPA_UP_TO_2250K_0
+#undef UCLBS_KAPPA_UP_TO_2250K_1
+#undef UCLBS_KAPPA_UP_TO_2250K_2
+#undef UCLBS_KAPPA_UP_TO_4250K_0
+#undef UCLBS_KAPPA_UP_TO_4250K_1
+#undef UCLBS_KAPPA_UP_TO_4250K_2
 
 }  // namespace uclbs

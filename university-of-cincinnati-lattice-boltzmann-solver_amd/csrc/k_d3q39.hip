@@ -428,7 +428,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     double dmu, dte;
     const double mu = sutherland39(T, gs, &dmu, &dte);
     double kappa = 0.0;
-    kerr = !therm_cond39(rho, T, gs, &kappa);
+    // FP64, plain lattice: uniform branches.  With a branch per lane hipcc (ROCm
+    // 7.2) put the copy of a live register (the interior launch's alpha status)
+    // ahead of the restore of the execution mask after it, so that nodes outside
+    // the conductivity fit were counted under a status that was not theirs.  The
+    // other variants' code has no such copy, and is 1% faster as it is.
+    if constexpr (!kFp32 && !kShifted) kerr = !therm_cond_wave39(rho, T, gs, &kappa);
+    else kerr = !therm_cond39(rho, T, gs, &kappa);
     double b1, b2;
     if (step < gs.startup) {
       b1 = gs.init_beta1 + gs.beta1_scale * (double)step;
