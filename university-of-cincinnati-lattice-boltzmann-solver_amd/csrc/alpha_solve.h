@@ -318,8 +318,10 @@ __device__ __forceinline__ void power_sums27(const double (&D)[27], const double
 }
 
 // alpha of an FP64 node from D_i, x_i = D_i / f_i, m = max|x|, xmin = min x.
-// The order of the series is the wavefront's (its largest m decides), so that
-// its lanes run one Newton; a lane beyond order 16 takes direct logarithms.
+// The lanes of a wavefront run one Newton on series of the largest order that
+// one of them needs; a lane that needs fewer terms has zeros for the others, so
+// that its alpha is its own order's to the bit, whatever its neighbours need.  A
+// lane beyond order 16 takes direct logarithms.
 __device__ __forceinline__ AlphaOut solve_alpha27(const double (&f)[27], const double (&D)[27],
                                                   const double (&x)[27], bool nonpos, double m,
                                                   double xmin, double alpha0, double tol, int maxit,
@@ -335,6 +337,10 @@ __device__ __forceinline__ AlphaOut solve_alpha27(const double (&f)[27], const d
     constexpr int N = decltype(order)::value;
     double S[N + 1];
     power_sums27<N>(D, x, S);
+    // products, not selects: around selects the compiler spills 300 registers
+    const double keep10 = m > thr.m7 ? 1.0 : 0.0, keep16 = m > thr.m10 ? 1.0 : 0.0;
+#pragma unroll
+    for (int n = 8; n <= N; ++n) S[n] *= n > 10 ? keep16 : keep10;
     const auto ev = series_poly<N>([&](int n) __attribute__((always_inline)) { return S[n]; });
     if (open && m <= thr.m16) r = newton_alpha(ev, S[2], amax, alpha0, tol, maxit);
   };
