@@ -24,6 +24,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "far_terms.h"
+
 namespace uclbs {
 
 enum : int { ALPHA_NEWTON = 0, ALPHA_TRIVIAL = 1, ALPHA_BOUND = 2, ALPHA_NONPOS = 3,
@@ -72,6 +74,13 @@ __device__ __forceinline__ double drcp(double v) {
   r = fma(fma(-v, r, 1.0), r, r);
   r = fma(fma(-v, r, 1.0), r, r);
   return r;
+}
+
+// 1/v for a value that is rounded to FP32 next: one Newton step on the estimate
+// (2^-23 or better), whose 2^-46 that rounding hides
+__device__ __forceinline__ double drcp_to_f32(double v) {
+  const double r = __builtin_amdgcn_rcp(v);
+  return r * (2.0 - v * r);
 }
 
 // ln(1 + x) for x > -1 in FP64, about 30 VALU operations: u = 1 + x = 2^e m
@@ -217,7 +226,8 @@ __device__ __forceinline__ AlphaOut newton_alpha(Eval&& ev, double S2, double am
 //   R = T_2 d^2 (|d| zmax)^(N-1) / (N (N+1) (1 - |d| zmax)).
 // One sweep (Q logarithms) gives g(a0), g'(a0) and T_2..T_N; Newton on the
 // order-N polynomial (scalar work) gives d, and a0 + d is the root when the
-// polynomial's residual plus R is within tol * S2.  Otherwise the next sweep
+// polynomial's residual plus R plus what the FP32 rounding of the T_n can add
+// (far_terms.h) is within tol * S2.  Otherwise the next sweep
 // is centred at a0 + d, kept inside the Newton bracket and within
 // |d| zmax <= 1/2.  From a seed near the root one sweep suffices where Newton
 // on direct logarithms evaluates g two to four times.  Bracket, bound and
@@ -226,13 +236,10 @@ __device__ __forceinline__ AlphaOut newton_alpha(Eval&& ev, double S2, double am
 // sweep(a, w, first) fills a Sweep; the first one also gives K = sum D ln(1 + x)
 // (every lane's first sweep is the same one, so that the branch is uniform).
 template <int N>
-struct Sweep {
+struct Sweep : FarTerms<N> {
   double K;
-  double g, gp;    // sum f ((1 + y) ln(1 + y) - y) and sum D ln(1 + y), y = a x
-  float zmax;      // max |z|
-  float T[N + 1];  // only steer the step (g and g' stay FP64 and decide
-                   // acceptance): FP32, their rounding in the bound below
-  bool edge;       // a at the positivity bound: some 1 + a x_i <= 0
+  double g, gp;  // sum f ((1 + y) ln(1 + y) - y) and sum D ln(1 + y), y = a x
+  bool edge;     // a at the positivity bound: some 1 + a x_i <= 0
 };
 template <int N, class SW>
 __device__ __forceinline__ AlphaOut recentred_alpha(SW&& sweep, double S2, double amax,
@@ -245,7 +252,7 @@ __device__ __forceinline__ AlphaOut recentred_alpha(SW&& sweep, double S2, doubl
   for (int k = 0;; ++k) {
     sweep(a, w, k == 0);
     const double g = fma(-a, w.K, w.g), gp = w.gp - w.K;
-    const double zmax = (double)w.zmax * (1.0 + 1e-6);  // not below the FP64 maximum
+    const double zmax = w.zbound();
     if (fabs(g) <= tol * S2) { r.alpha = a; r.iters = k; return r; }
     if (g < 0.0 && a >= amax) { r.alpha = amax; r.iters = k; r.status = ALPHA_BOUND; return r; }
     if (k >= maxit) { r.alpha = a; r.iters = k; r.status = ALPHA_NOCONV; return r; }
@@ -279,13 +286,7 @@ __device__ __forceinline__ AlphaOut recentred_alpha(SW&& sweep, double S2, doubl
 #pragma unroll
       for (int n = 0; n < N - 1; ++n) qp *= q;
       rem = (double)w.T[2] * dd * dd * qp * (1.0 / (N * (N + 1.0))) * drcp(1.0 - q);
-      // the FP32 coefficients: relative error below 1e-6 (27 terms summed),
-      // times the size of each polynomial term at dd
-      double terms = 0.0;
-#pragma unroll
-      for (int n = N; n >= 2; --n)
-        terms = fma(terms, fabs(dd), (double)fabsf(w.T[n]) * (1.0 / (n * (n - 1.0))));
-      rem = fma(1e-6 * dd * dd, terms, rem);
+      rem += w.slack(dd);
     }
     if (ok && fabs(p) + rem <= tol * S2) { r.alpha = a + dd; r.iters = k + 1; return r; }
     // next centre: the polynomial's step where it stays in the bracket and the

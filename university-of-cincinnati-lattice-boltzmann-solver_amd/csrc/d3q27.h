@@ -260,11 +260,9 @@ __device__ __forceinline__ AlphaOut collide27_far(float (&f)[27], double beta, c
         [&](double a, Sweep<kRecentreOrder>& w, bool first) __attribute__((always_inline)) {
           w.g = 0.0;
           w.gp = 0.0;
-          w.zmax = 0.0f;
           w.edge = false;
+          w.clear();
           if (first) w.K = 0.0;
-#pragma unroll
-          for (int n = 2; n <= kRecentreOrder; ++n) w.T[n] = 0.0f;
 #pragma unroll 3
           for (int i = 0; i < 27; ++i) {
             const float Di = sD[i * kFarBlock];
@@ -277,11 +275,7 @@ __device__ __forceinline__ AlphaOut collide27_far(float (&f)[27], double beta, c
             const double la = edge ? 0.0 : log1p_tab(y, lt);
             w.g = fma(fi, fma(A, la, -y), w.g);
             w.gp = fma(d, la, w.gp);
-            const float z = edge ? 0.0f : (float)x * frcp((float)A);
-            w.zmax = fmaxf(w.zmax, fabsf(z));
-            float t = Di;
-#pragma unroll
-            for (int n = 2; n <= kRecentreOrder; ++n) { t *= z; w.T[n] += t; }
+            w.add(Di, x, edge ? 0.0 : drcp_to_f32(A));
           }
         },
         S2, amax, seed, ac.tol, ac.maxit);

@@ -284,11 +284,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 
 // stores.  The queue length stays on the device; the blocks stride over the
 // queue, and those past its end leave once they have the lengths.  Block 0
 // zeroes the other set of lengths, which the next step appends to.
-// Bound by FP64 issue: a node takes ~3,200 operations (~27 x 75 of them in the
+// Bound by FP64 issue: a node takes ~3,300 operations (~27 x 77 of them in the
 // first sweep) and its queue is read and written once.  Blocks of two
 // wavefronts, five of them a CU by LDS; 2,560 blocks are two rounds of those.
-// 1.8M nodes a step on the 256^3 duct: 285 -> 252 us, 0.3M on the 149 x 77 x 61
-// duct: 70 -> 60 us, an empty queue 16 -> 5 us, against a grid of 32,768 blocks
+// 1.8M nodes a step on the 256^3 duct: 285 -> 259 us, 0.3M on the 149 x 77 x 61
+// duct: 70 -> 63 us, an empty queue 16 -> 5 us, against a grid of 32,768 blocks
 // of one wavefront, the sum K in a sweep of its own, quotients for reciprocals.
 // Two and eight lanes a node were slower (423, 528 us): the scalar part of the
 // root-find, a third of the work, is then repeated.
