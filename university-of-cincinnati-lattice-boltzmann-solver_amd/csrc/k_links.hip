@@ -242,6 +242,8 @@ __device__ int cast_wave(const LinkGeom& g, const double* e1, const double* e2, 
   F[2] = e1[0] * d[1] - e1[1] * d[0];
   const double near = 1e-2 * g.reach;
   const double clear = fmax(1e-12 * g.reach * g.reach, 4e-16 / near);
+  // lower beyond this and the plane at least near along the ray: upper > 4 kVSmall
+  const double steep = fmax(fmax(1.0e-9, 4.0 * kVSmall / near) * len, 4.0 * kPlusEps);
   // box_out over the segment's extremes
   auto inside = [&](const double* bb) __attribute__((always_inline)) {
     bool in = true;
@@ -281,8 +283,7 @@ __device__ int cast_wave(const LinkGeom& g, const double* e1, const double* e2, 
       const bool down = w[0] < -clear || w[1] > clear || w[2] < -clear;
       const bool sure = fabs(w[0]) > clear && fabs(w[1]) > clear && fabs(w[2]) > clear;
       const bool miss = up && down && sure && fabs(upper) * len >= near * fabs(lower) &&
-                        fabs(lower) > 1.0e-9 * len && fabs(upper - lower) > 1.0e-12 &&
-                        fabs(lower) > 4.0 * kPlusEps && fabs(upper) > 4.0 * kVSmall;
+                        fabs(lower) > steep && fabs(upper - lower) > 1.0e-12;
       if (!__any(in && !miss)) continue;
       if (in && !miss) {
         if (lower >= kMinusEps && lower <= kPlusEps) {
