@@ -5,7 +5,9 @@ The reference for a level of many boxes is the same region held as one box
 (itself checked against the oracle in test_gpu_d3q27 / test_gpu_amr): every
 node update is the same arithmetic on the same inputs, and ghost copies and
 injections are exact, so the fields must agree bit for bit, in FP64 and in
-FP32-shifted storage:
+FP32-shifted storage (these states stay in its order-6 tier; beyond it an FP32
+node's last bits follow the wavefront's order, see test_gpu_boxes_tiers.py for
+FP64):
   level 0 periodic domain split into uneven boxes == one periodic box;
   refined level split into uneven boxes == the same refined region as one box;
   hipGraph replays == eager launches, replay after replay with eager work and

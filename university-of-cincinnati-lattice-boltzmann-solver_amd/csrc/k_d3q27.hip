@@ -208,8 +208,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 
 // of one box), pulls over the box's strides -- a valid node's neighbours lie in
 // the box or its ghost shell -- and collides as k27_step_periodic does.  A
 // ghost node that shows a valid node s of the level (kFlagMirror) repeats s's
-// update -- the pull around s in s's box and the same collide, so the same
-// bits -- and stores it in place: the shell is current after the step with no
+// update -- the pull around s in s's box and the same collide: in FP64 the same
+// bits, in FP32 where both wavefronts take the same series order -- and stores it
+// in place: the shell is current after the step with no
 // copy pass (a deferred mirror is queued too, marked, and solved by the far
 // kernel like s).  Ghosts at a coarse-fine interface are interpolated before
 // the step.
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kShifted ? 
 // Bound by FP64 issue: a node takes ~3,300 operations (~27 x 77 of them in the
 // first sweep) and its queue is read and written once.  Blocks of two
 // wavefronts, five of them a CU by LDS; 2,560 blocks are two rounds of those.
-// 1.8M nodes a step on the 256^3 duct: 285 -> 259 us, 0.3M on the 149 x 77 x 61
+// 1.8M nodes a step on the 256^3 duct: 285 -> 256 us, 0.3M on the 149 x 77 x 61
 // duct: 70 -> 63 us, an empty queue 16 -> 5 us, against a grid of 32,768 blocks
 // of one wavefront, the sum K in a sweep of its own, quotients for reciprocals.
 // Two and eight lanes a node were slower (423, 528 us): the scalar part of the

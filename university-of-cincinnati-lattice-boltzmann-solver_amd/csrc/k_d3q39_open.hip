@@ -10,7 +10,7 @@
 // collision where it took 4,500.
 //
 // 65 x 48 x 33, FP32 storage: 116 -> 83 us a step; 96 x 80 x 64 shifted, FP64
-// storage: 861 -> 340 us (there g is not staged in LDS, so that four blocks fit
+// storage: 861 -> 350 us (there g is not staged in LDS, so that four blocks fit
 // a CU instead of two, and is read again ahead of alpha: 399 us where the
 // collision waited for it).  Distance from 64-bit results: 1.6e-9 as before, 1.4e-14
 // -> 1.2e-14.

@@ -44,8 +44,9 @@ __global__ __launch_bounds__(256) void k_fab_gather(const double* __restrict__ f
 // a dense FP64 copy (a second pass, a copy into the other buffer, and the
 // allocation of that copy on every call) import and export of a 256^3 D3Q27
 // level took 7.2 ms together where they take 2.4 ms in this form, and 20
-// steps between the two took 204 ms a pass, now 16.8 ms, when three contexts
-// took turns: their 3.6 GB allocations were returned and mapped anew each time.
+// steps between the two took 21.7 ms a pass, now 16.4 ms, and 204 ms when three
+// contexts took turns: their 3.6 GB allocations were returned and mapped anew
+// each time.
 template <typename S, int kGroup>
 __global__ __launch_bounds__(256) void k_fab_import(const double* __restrict__ fab, int ghost,
                                                     int64_t cstride, Box b, FabRef ref,
