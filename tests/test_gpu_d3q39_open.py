@@ -1,7 +1,7 @@
 """The periodic D3Q39 step at the boxes where it can go wrong: extents at the
 smallest that a level takes (the longest link is 4 on the shifted lattice), whole
 blocks and ragged ones; start-up ramps and past them; an iteration cap that
-leaves nodes unconverged.  FP64 against the oracle: 1e-11 relative (sums of 39
+leaves nodes unconverged; multipliers that are no numbers.  FP64 against the oracle: 1e-11 relative (sums of 39
 terms through 13 multipliers, 4 steps; measured below 1e-13)."""
 import numpy as np
 import pytest
@@ -54,3 +54,35 @@ def test_unconverged_nodes(pkg, orc, shifted, mach):
     for a, b in zip(out[0][0], out[1][0]):
         a, b = (v.reshape(-1, shape[2], shape[1], shape[0])[..., 4:-4] for v in (a, b))
         assert rel_l2(a, b) < 1e-11
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32s"])
+@pytest.mark.parametrize("shifted,mach", CASES)
+def test_nan_multipliers_are_reported(pkg, orc, shifted, mach, prec):
+    """A NaN among a node's multipliers leaves it without a real alpha root: the
+    step says so, with the number of such nodes (one in the first multiplier,
+    which stands in every exponent, counts as alpha = 2).  Their new populations
+    are NaN, the others as without it."""
+    shape = (12, 6, 5)
+    n = int(np.prod(shape))
+    c = orc.consts39(mach=mach, shifted=shifted)
+    f0, g0, lm0 = orc.init39(shape, *fields(shape, mach), c)
+    bad = np.arange(7, n, 11)
+    lm1 = lm0.reshape(13, n).copy()
+    lm1[np.arange(len(bad)) % 13, bad] = np.nan
+    first = int((np.arange(len(bad)) % 13 == 0).sum())
+    out = []
+    for lm in (lm0, lm1.reshape(lm0.shape)):
+        s = solver(pkg, shape, prec, mach, shifted)
+        s.upload_state(0, f0, g0, lm)
+        s.set_timestep(0, 60)
+        if lm is lm0:
+            s.step(0, 1)
+        else:
+            with pytest.raises(pkg.UclbsError, match=f": {len(bad) - first} nodes without a real alpha root"):
+                s.step(0, 1)
+            assert s.stats()["n_trivial"] == first
+        out.append(s.download_state(0)[0].reshape(39, n))
+    others = np.setdiff1d(np.arange(n), bad)
+    assert np.isnan(out[1][:, bad]).all()
+    assert np.array_equal(out[0][:, others], out[1][:, others])

@@ -54,7 +54,7 @@ __constant__ const double kExp2_64[64] = {
 // six bits the table's entry, the rest the exponent, e^r by its series (r^6 / 720
 // < 4e-17 relative): 12 FP64 operations where the general one takes over 20.
 // Within 1 ulp.  |x| is held below 2000, so that k fits and an overflow or an
-// underflow comes out of the exponent.
+// underflow comes out of the exponent.  (A NaN comes out as 0: see nan_status39.)
 struct ExpTab39 {
   const double* tab;  // kExp2_64 in LDS
   __device__ __forceinline__ double operator()(double x) const {
@@ -73,6 +73,19 @@ struct ExpTab39 {
     return ldexp(fma(b, q, b), k >> 6);
   }
 };
+
+// alpha's status where a multiplier is a NaN, else 0.  Multiplier 0 stands in
+// every exponent: no direction has an equilibrium, the estimate finds nothing to
+// sum (1: alpha = 2).  One of the others leaves some directions without: no real
+// root (-1), which the step reports.  Settled ahead of the iteration, as the
+// exponential above does not carry the NaN (a test of its argument costs each
+// exponential three operations) and the shifted lattice's change of basis spreads it.
+__device__ __forceinline__ int nan_status39(const double (&lm)[kM39]) {
+  bool nan = false;
+#pragma unroll
+  for (int k = 1; k < kM39; k += 2) nan |= __builtin_isunordered(lm[k], lm[k + 1]);
+  return lm[0] != lm[0] ? 1 : nan ? -1 : 0;
+}
 
 // exp(-s) for the argument left by a converged Newton's last update: its 13
 // entries are below 1e-7 and the monomials of one velocity add up to less than
@@ -208,6 +221,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
   __shared__ S sg[kStageG ? Q39 : 1][64];
   __shared__ double sd[Q39][64];
   __shared__ double etab[64];
+  __shared__ signed char nan_ast[64];  // kept here: Newton has no registers for it
   const int t = threadIdx.x;
   etab[t] = kExp2_64[t];
   __syncthreads();
@@ -272,6 +286,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
                              rho * (T + u[1] * u[1]), rho * (T + u[2] * u[2]), rho * u[0] * u[1],
                              rho * u[0] * u[2], rho * u[1] * u[2], qf * u[0], qf * u[1],
                              qf * u[2]};
+    if (kTurb) nan_ast[t] = (signed char)nan_status39(lm);
     double dp[kM39];
     // the last iteration's equilibrium stays in LDS for alpha and collision
     const ExpTab39 ex{etab};
@@ -289,7 +304,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     double dim_mu, dim_temp;
     const double mu = sutherland_open39(T, gs, &dim_mu, &dim_temp);
     double al = 2.0;
-    if (kTurb) al = alpha_open39<kShifted>(sf, sd, t, rf, dim_mu, dim_temp, step, gs, &ast);
+    if (kTurb) {
+      al = alpha_open39<kShifted>(sf, sd, t, rf, dim_mu, dim_temp, step, gs, &ast);
+      const int na = nan_ast[t];
+      ast = na ? na : ast;
+      al = na ? 2.0 : al;
+    }
     if (kKeepAlpha) alpha[node] = al;
 
     // collision: deviation d from the updated multipliers' equilibrium,
